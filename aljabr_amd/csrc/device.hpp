@@ -279,4 +279,31 @@ __device__ __forceinline__ float nf4_level_sel(int c) {
     return v;
 }
 
+// LDS-DMA loads (global_load_lds: 16 bytes per lane, landing at
+// `lds_base` + 16 * lane). Written as inline assembly: the compiler models
+// the builtin like a FLAT access that also counts on the LDS counter and
+// then waits for every outstanding LDS read before using any of them, which
+// would serialize the table lookups; the hardware counts these loads on the
+// vector-memory counter only, and every wait for their data here is an
+// explicit vmcnt. M0 carries the LDS address (latched at issue, one wait
+// state after it is written) and is restored afterwards.
+__device__ __forceinline__ void dma16(const void *g, uint32_t lds_base) {
+    uint32_t save;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\t"
+                 "s_mov_b32 m0, %0"
+                 : "=&s"(save)
+                 : "s"(lds_base), "v"(g)
+                 : "memory");
+}
+
+// The 4-byte form of dma16.
+__device__ __forceinline__ void dma4(const void *g, uint32_t lds_base) {
+    uint32_t save;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %2, off\n\t"
+                 "s_mov_b32 m0, %0"
+                 : "=&s"(save)
+                 : "s"(lds_base), "v"(g)
+                 : "memory");
+}
+
 }  // namespace aljabr

@@ -62,6 +62,19 @@ int enqueue_matmul_multi(float *const *C, const float *A, const uint8_t *const *
         if (enqueue_rows_fused(type[0], outs, n, A, nullptr, 0.0f, K, 0, kRowsStore) == ALJABR_ROCM_OK)
             return ALJABR_ROCM_OK;
     }
+    if (same && prompt_gguf(type[0], batch, N[0], K)) {
+        RowsOut outs[3];
+        const int xparts = prompt_xparts(type[0], N[0], K);
+        bool stack = true;                       // one precision for the stack
+        for (int i = 0; i < n; ++i) {
+            outs[i] = RowsOut{C[i], B[i], nullptr, N[i]};
+            stack = stack && prompt_gguf(type[0], batch, N[i], K) && prompt_xparts(type[0], N[i], K) == xparts;
+        }
+        if (stack) {
+            const int rc = enqueue_prompt_gemm(outs, n, A, K, type[0], xparts, batch);
+            if (rc != ALJABR_ROCM_ERR_UNSUPPORTED) return rc;
+        }
+    }
     if (same && batch >= 2 && kquant_mfma_type(type[0]) && batch <= kquant_mfma_max_m(type[0])) {
         KqOut outs[3];
         for (int i = 0; i < n; ++i) outs[i] = KqOut{C[i], B[i], N[i]};

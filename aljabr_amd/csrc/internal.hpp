@@ -41,6 +41,9 @@ int finish_launch(const char *what);
 constexpr int kScratchSlots = 2;
 constexpr int kScratchPartials = 1;
 void *stream_scratch(size_t bytes, int slot = 0);
+// The same for a caller that has another way to do the work: nullptr without
+// an error recorded.
+void *stream_scratch_try(size_t bytes, int slot);
 // Bytes of stream scratch held for the calling thread's stream (all slots).
 size_t stream_scratch_held();
 

@@ -219,6 +219,21 @@ int enqueue_nf4_mfma_multi(const RowsOut *outs, int nseg, const float *A, int K,
                            const uint16_t *xpacked = nullptr);
 // Bytes of the fp16 A image for M <= 64 tokens over K (K % 64 == 0).
 size_t nf4_xpack_bytes(int M, int K);
+// C = A . W^T for prompts (prompt_gemm.hip): up to three stacked matrices of
+// one type (NF4 with block size 64, Q4_0, Q8_0, Q4_K, Q6_K; all but the last
+// with a multiple of 32 rows), the activations as `xparts` fp16 parts (1:
+// rounded once, NF4 and Q4_K only; 2: hi and lo). The image and the K slices'
+// partials live in the stream's scratch. ALJABR_ROCM_ERR_UNSUPPORTED (nothing
+// enqueued) when the shape does not fit or the scratch cannot be had (under
+// capture).
+int enqueue_prompt_gemm(const RowsOut *outs, int nseg, const float *A, int K, int type, int xparts, int M);
+// Whether the passes of up to 32 tokens round the activations of a Q4_K
+// matrix to fp16 (q4k_gemm_pass takes its shape).
+bool q4k_rounds_activations(int N, int K);
+// Whether M tokens of a GGUF type are a prompt, and the activation parts its
+// GEMM takes (those of the passes it replaces).
+bool prompt_gguf(int type, int M, int N, int K);
+int prompt_xparts(int type, int N, int K);
 // GGUF Q4_0 / Q8_0 GEMM pass of M <= 16 tokens with the activations held in
 // registers (K % 2048 == 0, A 16-byte aligned; up to three stacked matrices
 // of one type, all but the last a multiple of 16 rows; fp32-accurate,

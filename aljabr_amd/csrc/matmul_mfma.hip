@@ -34,6 +34,7 @@
 // Determinism. With several K slices, each workgroup stores its partial
 // tile and a second kernel sums the slices in slice order into Y (or adds
 // them to it): no float atomics, the same result on every run.
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -680,31 +681,6 @@ __device__ __forceinline__ void wait_tiles(int n) {
         else
             wait_tiles<KD, J - 1>(n);
     }
-}
-
-// LDS-DMA loads (global_load_lds: 16 or 4 bytes per lane, landing at
-// `lds_base` + size * lane). Written as inline assembly: the compiler models
-// the builtin like a FLAT access that also counts on the LDS counter and
-// then waits for every outstanding LDS read before using any of them, which
-// would serialize the table lookups; the hardware counts these loads on the
-// vector-memory counter only, and every wait for their data here is an
-// explicit vmcnt. M0 carries the LDS address (latched at issue, one wait
-// state after it is written) and is restored afterwards.
-__device__ __forceinline__ void dma16(const void *g, uint32_t lds_base) {
-    uint32_t save;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\t"
-                 "s_mov_b32 m0, %0"
-                 : "=&s"(save)
-                 : "s"(lds_base), "v"(g)
-                 : "memory");
-}
-__device__ __forceinline__ void dma4(const void *g, uint32_t lds_base) {
-    uint32_t save;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %2, off\n\t"
-                 "s_mov_b32 m0, %0"
-                 : "=&s"(save)
-                 : "s"(lds_base), "v"(g)
-                 : "memory");
 }
 
 // LDS-DMA loads of one tile (this wave's K range of rows 16t .. 16t+15) into
@@ -1722,6 +1698,14 @@ int q4k_gemm_pass(const RowsOut *outs, int nseg, const float *A, int K, int M, b
     if (tail) return enqueue_slice_tail(*tail, args.part, slices, M, args.N);
     if (slices > 1) return enqueue_slice_sum(args.y, args.end, nseg, M, args.N, args.part, slices, add);
     return ALJABR_ROCM_OK;
+}
+
+bool q4k_rounds_activations(int N, int K) {
+    if (K % 4096 != 0 || N < 1) return false;
+    const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
+    const int tiles = (N + 15) / 16;
+    const int gr = std::min(std::max(cus / (K / 4096), 1), tiles);
+    return (tiles + gr - 1) / gr >= 3;
 }
 
 size_t q4k_gemm_scratch_floats(int M, int N, int K) {

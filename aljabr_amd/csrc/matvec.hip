@@ -458,6 +458,30 @@ using namespace aljabr;
 
 namespace aljabr {
 
+// Where the prompt GEMM (a pass over the weights to lay them out, then one
+// for all tokens) beats the passes of 8, 32 or 64 tokens, in us per FFN of
+// three matrices, passes against prompt GEMM:
+//   Q4_0/Q8_0 1024 x 2816    12 tokens 56/34;  2560 x 7680 12: 90/68;
+//             4096 x 14336   16: 112/132, 24: 168/133
+//   Q4_K/Q6_K 1024 x 2816    33: 93/42;  2560 x 7680 (Q6_K) 33: 99/93;
+//             4096 x 14336   48: 145/144, 65: 193/182;
+//             Q/K/V of 1024  33: 35/48, 128: 105/50 (three small launches)
+//   NF4       1024 x 2816    128: 64/64, 192: 95/70;  2048 x 5632 129: 127/97;
+//             4096 x 14336   129: 222/228, 192: 268/243
+//             2560 x 7680    65: 129/102 (the passes split the activations)
+static constexpr long long kLargeMatrix = 32LL << 20, kSmallMatrix = 2LL << 20;   // N * K
+
+bool prompt_gguf(int type, int M, int N, int K) {
+    const long long size = static_cast<long long>(N) * K;
+    if (type == ALJABR_ROCM_TYPE_Q4_K || type == ALJABR_ROCM_TYPE_Q6_K)
+        return M > (size >= kLargeMatrix || size < kSmallMatrix ? 64 : 32);
+    return (type == ALJABR_ROCM_TYPE_Q4_0 || type == ALJABR_ROCM_TYPE_Q8_0) && M > (size >= kLargeMatrix ? 16 : 8);
+}
+
+static bool prompt_nf4(int M, int N, int K) {
+    return M > (K % 1024 != 0 ? 64 : static_cast<long long>(N) * K >= kLargeMatrix ? 144 : 128);
+}
+
 // M > 8 slices run the small-M kernels per slice of 8 tokens (weights are
 // re-read per slice); the MFMA path takes over at its threshold.
 int enqueue_matmul_nf4(float *C, const float *A, const uint8_t *Bq, const float *absmax, int K, int N, int bs, int M,
@@ -467,6 +491,13 @@ int enqueue_matmul_nf4(float *C, const float *A, const uint8_t *Bq, const float 
         const int shift = log2_exact(bs);
         if (shift >= 0 && enqueue_rows_nf4_mt(C, A, Bq, absmax, K, N, shift, M) == ALJABR_ROCM_OK)
             return ALJABR_ROCM_OK;
+    }
+    // Prompts (without a session's own buffer): the weights once for all
+    // tokens instead of once per 64.
+    if (!part && bs == 64 && aligned(Bq, 16) && prompt_nf4(M, N, K)) {
+        const RowsOut o{C, Bq, absmax, N};
+        const int rc = enqueue_prompt_gemm(&o, 1, A, K, ALJABR_ROCM_TYPE_NF4, K % 1024 == 0 ? 1 : 2, M);
+        if (rc != ALJABR_ROCM_ERR_UNSUPPORTED) return rc;
     }
     // M >= 2 on the matrix cores when the shape allows (deterministic;
     // passes of 64 tokens).
@@ -484,8 +515,17 @@ int enqueue_matmul_nf4(float *C, const float *A, const uint8_t *Bq, const float 
     return ALJABR_ROCM_OK;
 }
 
+int prompt_xparts(int type, int N, int K) {
+    return type == ALJABR_ROCM_TYPE_Q4_K && q4k_rounds_activations(N, K) ? 1 : 2;
+}
+
 int enqueue_matmul_gguf(float *C, const float *A, const uint8_t *B, int K, int N, int type, int M, float *part,
                         size_t part_floats) {
+    if (!part && prompt_gguf(type, M, N, K)) {
+        const RowsOut o{C, B, nullptr, N};
+        const int rc = enqueue_prompt_gemm(&o, 1, A, K, type, prompt_xparts(type, N, K), M);
+        if (rc != ALJABR_ROCM_ERR_UNSUPPORTED) return rc;
+    }
     if (type == ALJABR_ROCM_TYPE_Q4_K || type == ALJABR_ROCM_TYPE_Q6_K)
         return enqueue_matmul_kquant(C, A, B, K, N, type, M, part, part_floats);
     // Q4_0 / Q8_0 with M >= 2 on the matrix cores (K % 512, 16-byte aligned),

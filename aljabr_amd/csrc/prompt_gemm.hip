@@ -1,0 +1,229 @@
+// prompt_gemm.hip - the prompt GEMM's activation image, plan and dispatch
+// (the kernels: prompt_gemm.hpp and prompt_{nf4,q40,q80,q4k,q6k}.hip).
+#include <algorithm>
+
+#include "prompt_gemm.hpp"
+
+namespace aljabr {
+namespace {
+
+using pg::half8;
+
+// The activations as A fragments: [chunk kb][32-token tile][step j][lane] of
+// 8 fp16, lane l = 32h + i holding token 32*tile + i, elements 64kb + 16j +
+// 8h + e (NF4 order: 64kb + 32h + 8j + e), zero past M and K; hi = fp16(x)
+// and, with xl, lo = fp16(x - hi). One workgroup per (chunk, tile), one wave
+// per step. With sums (Q4_K): the sums of each 32-element sub-block of what
+// the parts hold, split hi / lo (lane half 0 / 1), [super-block][tile][lane]
+// of 8 sub-blocks.
+__global__ __launch_bounds__(256) void prompt_pack_kernel(const float *x, u32x4 *xh, u32x4 *xl, _Float16 *sums, int M,
+                                                          int K, int tiles, int nf4, const float *scale) {
+    __shared__ float part[4][64];
+    const int tid = threadIdx.x, lane = tid & 63, j = tid >> 6, h = lane >> 5, i = lane & 31;
+    const int tile = blockIdx.x % tiles, kb = blockIdx.x / tiles;
+    const int m = 32 * tile + i;
+    const int k = 64 * kb + (nf4 ? 32 * h + 8 * j : 16 * j + 8 * h);
+    float4 a = {0.0f, 0.0f, 0.0f, 0.0f}, b = a;
+    if (m < M && k < K) {                            // K % 32 == 0: the 8 elements are in or out together
+        const float4 *src = reinterpret_cast<const float4 *>(x + static_cast<size_t>(m) * K + k);
+        a = src[0];
+        b = src[1];
+    }
+    float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    if (scale && m < M) {
+        const float inv = 1.0f / scale[m];           // powers of two: exact
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] *= inv;
+    }
+    half8 hi, lo;
+    float t = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        hi[e] = static_cast<_Float16>(v[e]);
+        lo[e] = isinf(static_cast<float>(hi[e])) ? static_cast<_Float16>(0.0f)
+                                                 : static_cast<_Float16>(v[e] - static_cast<float>(hi[e]));
+        t += xl ? v[e] : static_cast<float>(hi[e]);
+    }
+    const size_t at = (static_cast<size_t>(blockIdx.x) * 4 + j) * 64 + lane;
+    xh[at] = __builtin_bit_cast(u32x4, hi);
+    if (xl) xl[at] = __builtin_bit_cast(u32x4, lo);
+    if (!sums) return;
+    part[j][lane] = t;
+    __syncthreads();
+    if (tid < 64) {
+        const int sb = tid >> 5;                     // sub-block of the chunk: steps 2sb and 2sb + 1
+        const float s = (part[2 * sb][i] + part[2 * sb][32 + i]) + (part[2 * sb + 1][i] + part[2 * sb + 1][32 + i]);
+        const _Float16 sh = static_cast<_Float16>(s);
+        _Float16 *dst = sums + ((static_cast<size_t>(kb >> 2) * tiles + tile) * 64 + i) * 8 + 2 * (kb & 3) + sb;
+        dst[0] = sh;
+        dst[32 * 8] = static_cast<_Float16>(s - static_cast<float>(sh));
+    }
+}
+
+// The plan's constants are fits of a sweep over tiles, slices and formats
+// (4096 x 14336 and 2560-wide layers, 64 to 2048 tokens): a chunk of four
+// token tiles took 1.65 us for two products (NF4, Q8_0), 2.4 us for Q6_K's
+// three; the slice sum moves ~5 TB/s.
+constexpr int kPassTokens = 4096;                    // bounds the activation image
+constexpr float kPartialMb = 128.0f;                  // bounds the K slices' partial sums
+// The power of two that brings a token row's largest finite magnitude into
+// [2^8, 2^9): with it any fp32 row fits the fp16 parts. One workgroup a row.
+__global__ __launch_bounds__(256) void prompt_scale_kernel(const float *x, float *scale, int K) {
+    __shared__ float best[4];
+    const float *row = x + static_cast<size_t>(blockIdx.x) * K;
+    float top = 0.0f;
+    for (int k = threadIdx.x; k < K; k += 256) {
+        const float v = fabsf(row[k]);
+        if (v <= 3.4028235e38f) top = fmaxf(top, v);
+    }
+    top = wave_max(top);
+    if ((threadIdx.x & 63) == 0) best[threadIdx.x >> 6] = top;
+    __syncthreads();
+    if (threadIdx.x) return;
+    top = fmaxf(fmaxf(best[0], best[1]), fmaxf(best[2], best[3]));
+    int e = 9;
+    if (top > 0.0f) (void)frexpf(top, &e);           // top in [2^(e-1), 2^e)
+    scale[blockIdx.x] = ldexpf(1.0f, (e < -100 ? -100 : e) - 9);
+}
+
+constexpr size_t kPanelBytes = size_t{128} << 20;     // bounds the weight image
+constexpr float kFixedUs = 3.0f, kReduceUs = 3.0f, kMbPerUs = 5.0f;
+
+// Tiles of 32 tokens per wave (2 or 4) and K slices for M tokens over N
+// stacked rows. Two tiles leave less idle in the last token group, four
+// decode and read the weights half as often.
+//
+// K slices trade idle CUs and ragged last rounds against the partial sums'
+// traffic: the least of rounds * (chunks * chunk time + fixed) + slice sum.
+struct Plan {
+    int mt, mt_groups, n_groups, per, slices;
+};
+
+Plan make_plan(int f, int xp, int M, int N, int chunks, int cus) {
+    const int quantum = f == kPgQ4K || f == kPgQ6K ? 4 : 1;
+    // Microseconds of a workgroup's chunk: 32 cycles per product and its share
+    // of the decode and the scaling.
+    const float products = f == kPgQ6K ? 3.0f : f == kPgQ4K ? 1.12f * xp : f == kPgNF4 ? 1.0f + xp : 2.0f;
+    Plan best{};
+    float best_us = 0.0f;
+    const float out_mb = 4e-6f * static_cast<float>(M) * static_cast<float>(N);
+    const int n_groups = (N + 64 * kPgWaves - 1) / (64 * kPgWaves);
+    for (int mt = 4; mt >= 2; mt -= 2) {
+        const float chunk_us = (0.4f + 0.68f * products) * (mt == 4 ? 1.0f : 0.55f);
+        const int mt_groups = (M + 32 * mt - 1) / (32 * mt);
+        for (int s = 1; s <= 32; ++s) {
+            if (s > 1 && (s * out_mb > kPartialMb || chunks / s < quantum)) break;
+            Plan p{mt, mt_groups, n_groups, 0, 0};
+            p.per = (chunks + s - 1) / s;
+            p.per = (p.per + quantum - 1) / quantum * quantum;
+            p.slices = (chunks + p.per - 1) / p.per;
+            const long long rounds = (static_cast<long long>(mt_groups) * n_groups * p.slices + cus - 1) / cus;
+            const float us = static_cast<float>(rounds) * (static_cast<float>(p.per) * chunk_us + kFixedUs) +
+                             (p.slices > 1 ? kReduceUs + static_cast<float>(2 * p.slices + 1) * out_mb / kMbPerUs : 0.0f);
+            if (best_us == 0.0f || us < best_us) {
+                best = p;
+                best_us = us;
+            }
+        }
+    }
+    return best;
+}
+
+}  // namespace
+
+int enqueue_prompt_gemm(const RowsOut *outs, int nseg, const float *A, int K, int type, int xparts, int M) {
+    const int f = type == ALJABR_ROCM_TYPE_NF4    ? kPgNF4
+                  : type == ALJABR_ROCM_TYPE_Q4_0 ? kPgQ40
+                  : type == ALJABR_ROCM_TYPE_Q8_0 ? kPgQ80
+                  : type == ALJABR_ROCM_TYPE_Q4_K ? kPgQ4K
+                  : type == ALJABR_ROCM_TYPE_Q6_K ? kPgQ6K
+                                                  : -1;
+    const int block = f == kPgNF4 ? 64 : f == kPgQ40 || f == kPgQ80 ? 32 : 256;
+    if (f < 0 || nseg < 1 || nseg > 3 || M < 2 || K < block || K % block != 0 || !aligned(A, 16) || !mfma_enabled())
+        return ALJABR_ROCM_ERR_UNSUPPORTED;
+    PgArgs a{};
+    long long end = 0;
+    for (int i = 0; i < 3; ++i) {
+        a.end[i] = 0x7fffffff;
+        if (i >= nseg) continue;
+        const RowsOut &o = outs[i];
+        const size_t wa = f == kPgNF4 || f == kPgQ4K ? 16 : 4;
+        if (o.n <= 0 || !aligned(o.w, wa) || (i < nseg - 1 && o.n % 32 != 0)) return ALJABR_ROCM_ERR_UNSUPPORTED;
+        end += o.n;
+        if (end > 0x7fff0000LL) return ALJABR_ROCM_ERR_UNSUPPORTED;
+        a.w[i] = o.w;
+        a.absmax[i] = o.absmax;
+        a.end[i] = static_cast<int>(end);
+    }
+    // Shapes whose passes compute in fp32 (they are not the matrix-core
+    // kernels') keep fp32's range: their rows are scaled.
+    const bool scaled = xparts == 2 && K % (f == kPgNF4 ? 256 : 512) != 0;
+    a.nseg = nseg;
+    a.N = static_cast<int>(end);
+    a.K = K;
+    a.chunks = (K + kPgChunk - 1) / kPgChunk;
+    const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
+    hipStream_t s = current_stream();
+    // Weight image bytes of a row tile, and the panels that bound it.
+    const size_t tile_codes = static_cast<size_t>(a.chunks) * (f == kPgQ80 || f == kPgQ6K ? 2048 : 1024);
+    const size_t tile_aux = static_cast<size_t>(a.chunks) * (f == kPgQ6K ? 256 : 128) +
+                            (f == kPgQ4K ? static_cast<size_t>(a.chunks / 4) * pg::kMinWords * 4 : 0);
+    const int all_tiles = (a.N + 31) / 32;
+    const int panels = static_cast<int>((all_tiles * (tile_codes + tile_aux) + kPanelBytes - 1) / kPanelBytes);
+    const int panel = (all_tiles + panels - 1) / panels;
+    for (int m0 = 0; m0 < M; m0 += kPassTokens) {
+        const int mm = std::min(M - m0, kPassTokens);
+        const Plan p = make_plan(f, xparts, mm, std::min(panel * 32, a.N), a.chunks, cus);
+        a.M = mm;
+        a.per = p.per;
+        a.slices = p.slices;
+        a.mt_groups = p.mt_groups;
+        a.tiles = p.mt_groups * p.mt;
+        const size_t plane = static_cast<size_t>(a.chunks) * a.tiles * 4096;
+        const size_t sums = f == kPgQ4K ? static_cast<size_t>(a.chunks / 4) * a.tiles * 1024 : 0;
+        const size_t image = (panel * (tile_codes + tile_aux) + 255) & ~size_t{255};
+        const size_t scales = scaled ? (static_cast<size_t>(mm) * sizeof(float) + 255) & ~size_t{255} : 0;
+        const size_t parts = p.slices > 1 ? static_cast<size_t>(p.slices) * mm * a.N * sizeof(float) : 0;
+        uint8_t *buf =
+            static_cast<uint8_t *>(stream_scratch_try(xparts * plane + sums + image + scales + parts, kScratchPartials));
+        if (!buf) return m0 == 0 ? ALJABR_ROCM_ERR_UNSUPPORTED : ALJABR_ROCM_ERR_BUFFER;
+        uint8_t *xl = xparts == 2 ? buf + plane : nullptr;
+        uint8_t *next = buf + xparts * plane;
+        a.xh = buf;
+        a.xl = xl;
+        a.sums = sums ? next : nullptr;
+        a.codes = next + sums;
+        float *scale = scaled ? reinterpret_cast<float *>(next + sums + image) : nullptr;
+        a.scale = scale;
+        a.part = parts ? reinterpret_cast<float *>(next + sums + image + scales) : nullptr;
+        for (int i = 0; i < nseg; ++i) a.y[i] = outs[i].y + static_cast<size_t>(m0) * outs[i].n;
+        const float *x = A + static_cast<size_t>(m0) * K;
+        if (scaled) hipLaunchKernelGGL(prompt_scale_kernel, dim3(mm), dim3(256), 0, s, x, scale, K);
+        hipLaunchKernelGGL(prompt_pack_kernel, dim3(static_cast<unsigned>(a.chunks * a.tiles)), dim3(256), 0, s,
+                           x, reinterpret_cast<u32x4 *>(buf),
+                           reinterpret_cast<u32x4 *>(xl),
+                           reinterpret_cast<_Float16 *>(const_cast<uint8_t *>(a.sums)), mm, K, a.tiles, f == kPgNF4,
+                           static_cast<const float *>(scale));
+        for (a.tile0 = 0; a.tile0 < all_tiles; a.tile0 += panel) {
+            a.ntiles = std::min(panel, all_tiles - a.tile0);
+            a.n_groups = (a.ntiles + 2 * kPgWaves - 1) / (2 * kPgWaves);
+            a.aux = reinterpret_cast<const uint32_t *>(a.codes + a.ntiles * tile_codes);
+            int rc = ALJABR_ROCM_OK;
+            switch (f) {
+            case kPgNF4: rc = prompt_launch_nf4(a, xparts, p.mt, s); break;
+            case kPgQ40: rc = prompt_launch_q40(a, p.mt, s); break;
+            case kPgQ80: rc = prompt_launch_q80(a, p.mt, s); break;
+            case kPgQ4K: rc = prompt_launch_q4k(a, xparts, p.mt, s); break;
+            default: rc = prompt_launch_q6k(a, p.mt, s); break;
+            }
+            if (rc != ALJABR_ROCM_OK) return rc;
+        }
+        if (a.part) {
+            const int rc = enqueue_slice_sum(a.y, a.end, nseg, mm, a.N, a.part, p.slices, false);
+            if (rc != ALJABR_ROCM_OK) return rc;
+        }
+    }
+    return ALJABR_ROCM_OK;
+}
+
+}  // namespace aljabr

@@ -140,6 +140,18 @@ void *stream_scratch(size_t bytes, int slot) {
     return p;
 }
 
+void *stream_scratch_try(size_t bytes, int slot) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(current_stream(), &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return nullptr;
+    const std::string error = tls().error;
+    void *p = stream_scratch(bytes, slot);
+    if (!p) {
+        tls().error = error;
+        (void)hipGetLastError();                 // the caller goes on without the buffer
+    }
+    return p;
+}
+
 size_t stream_scratch_held() {
     Context &c = ctx();
     const hipStream_t s = current_stream();

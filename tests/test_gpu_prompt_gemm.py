@@ -1,0 +1,83 @@
+"""GPU parity of the prompt GEMM (matmuls of more tokens than one pass of the
+small-M kernels): every format at the edges of its tiles (32 tokens x 32 rows
+a tile, 64 or 128 tokens and 256 rows a workgroup, 64-element chunks), against
+the oracle. Tolerances: two fp16 activation parts carry 2^-22 an element, so
+the fp32 sums' 2^-24 * sqrt(K) dominate and 2e-6 of a row holds with room. One
+part (NF4 at K % 1024 == 0, Q4_K at the shapes whose passes round) is fp16(x)
+times the exact weights: the reference multiplies fp16(x), so the same bound
+holds (against x itself the rounding is 2^-12 of |w||x|, whatever cancels in
+the row)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from conftest import rel_l2
+
+pytestmark = pytest.mark.gpu
+Q4_0, Q8_0, Q4_K, Q6_K = 2, 8, 12, 14
+TOL = 2e-6
+
+
+def _weights(oracle, t, n, k, seed):
+    if t in (Q4_K, Q6_K):
+        return oracle.random_k_blocks(t, n * k // 256, seed, scale=0.5 / np.sqrt(k) / (200 if t == Q4_K else 1000))
+    return oracle.quantize(t, oracle.normal(seed, n * k, 0.0, 0.5 / np.sqrt(k)))
+
+
+def _decoded(oracle, t, raw, n, k):
+    return oracle.dequant(t, raw, n * k).reshape(n, k).astype(np.float64)
+
+
+def _parts(x, rounded):
+    return (x.astype(np.float16) if rounded else x).astype(np.float64)
+
+
+@pytest.mark.parametrize("t,n,k,m", [
+    (Q4_0, 33, 32, 9), (Q4_0, 257, 1056, 65), (Q4_0, 64, 512, 128), (Q4_0, 300, 2048, 129),
+    (Q8_0, 1, 96, 17), (Q8_0, 255, 640, 64), (Q8_0, 512, 2560, 197), (Q8_0, 31, 1024, 33),
+    (Q4_K, 33, 256, 65), (Q4_K, 1000, 2304, 66), (Q4_K, 12300, 4096, 130), (Q4_K, 257, 4096, 300),
+    (Q6_K, 7, 256, 65), (Q6_K, 1024, 2560, 97), (Q6_K, 300, 1280, 257)])
+def test_gguf_prompt(rocm, dev, oracle, t, n, k, m):
+    raw = _weights(oracle, t, n, k, 3)
+    x = oracle.normal(4, m * k).reshape(m, k)
+    x[1] *= 3e4 if k % 512 else 1.0          # past fp16's range: these shapes take any fp32 row
+    y = dev.empty(m * n)
+    w, xd = dev.put(raw), dev.put(x)
+    rocm.call("aljabr_rocm_matvec_tb_batch", dev.ptr(y), dev.ptr(xd), dev.ptr(w), k, n, t, m)
+    got = dev.get(y).reshape(m, n)
+    rounded = t == Q4_K and k == 4096 and n > 8192
+    ref = _parts(x, rounded) @ _decoded(oracle, t, raw, n, k).T
+    for i in range(m):
+        assert rel_l2(got[i], ref[i]) <= TOL, i
+
+
+@pytest.mark.parametrize("n,k,m", [(33, 192, 65), (257, 1280, 66), (300, 1024, 129), (2048, 2048, 256), (64, 4096, 145)])
+def test_nf4_prompt(rocm, dev, oracle, n, k, m):
+    codes, absmax = oracle.nf4_quantize(oracle.normal(5, n * k, 0.0, 0.02), 64)
+    x = oracle.normal(6, m * k).reshape(m, k)
+    y = dev.empty(m * n)
+    c, a, xd = dev.put(codes), dev.put(absmax), dev.put(x)
+    rocm.call("aljabr_rocm_matvec_tb_batch_nf4", dev.ptr(y), dev.ptr(xd), dev.ptr(c), dev.ptr(a), k, n, 64, m)
+    got = dev.get(y).reshape(m, n)
+    ref = _parts(x, k % 1024 == 0) @ oracle.nf4_dequant(codes, absmax, n * k, 64).reshape(n, k).astype(np.float64).T
+    for i in range(m):
+        assert rel_l2(got[i], ref[i]) <= TOL, i
+
+
+@pytest.mark.parametrize("t,ns,k,m", [(Q8_0, (320, 64, 33), 640, 100), (Q4_K, (2048, 1024, 1056), 1024, 65),
+                                      (Q4_0, (96, 32, 32), 1024, 40)])
+def test_stacked_prompt(rocm, dev, oracle, t, ns, k, m):
+    """Three matrices in one launch equal the oracle; repeats are identical."""
+    raws = [_weights(oracle, t, n, k, 20 + i) for i, n in enumerate(ns)]
+    x = oracle.normal(8, m * k).reshape(m, k)
+    ws, xd = [dev.put(r) for r in raws], dev.put(x)
+    outs = []
+    for _ in range(2):
+        ys = [dev.empty(m * n) for n in ns]
+        rocm.call("aljabr_rocm_matvec_tb_triple_batch", *[dev.ptr(y) for y in ys], dev.ptr(xd),
+                  *[dev.ptr(w) for w in ws], k, *ns, t, t, t, m)
+        outs.append([dev.get(y).reshape(m, n) for y, n in zip(ys, ns)])
+    for got, again, raw, n in zip(*outs, raws, ns):
+        assert np.array_equal(got, again)
+        assert rel_l2(got, x.astype(np.float64) @ _decoded(oracle, t, raw, n, k).T) <= TOL
