@@ -615,6 +615,13 @@ int launch_paged(const AttnParams &p, int G, int splits, int chunk, float *part,
 
 }  // namespace
 
+void enqueue_attention_merge(const AttnParams &p, const float *part_o, const float *part_ml, int splits) {
+    const unsigned rows = static_cast<unsigned>(p.B * p.Hq * p.Sq);
+    const auto fn = p.D == 64 ? attn_merge_kernel<64> : attn_merge_kernel<128>;
+    hipLaunchKernelGGL(fn, dim3(rows), dim3(256), 0, current_stream(), part_o, part_ml, p.out, splits, p.Sq, p.Hq,
+                       p.Hq * p.Sq * p.D, p.Sq * p.D, p.D, p.norm_eps, static_cast<uint16_t *>(nullptr));
+}
+
 // Chunks hold at least 64 keys (rounded to 16), so there are at most
 // ceil(keys / 64) + 1 splits.
 size_t attention_scratch_bytes(int B, int Hq, int Sq, int D, int keys) {
@@ -732,7 +739,8 @@ extern "C" int aljabr_rocm_attention_gqa(void *out, const void *Q, const void *K
     p.scale = scale > 0.0f ? scale : static_cast<float>(1.0 / std::sqrt(static_cast<double>(D)));
     p.causal = causal != 0;
     p.kv_f16 = kvType == ALJABR_ROCM_TYPE_F16;
-    int rc = enqueue_attention(p);
+    int rc = enqueue_attention_chunk(p);
+    if (rc == ALJABR_ROCM_ERR_UNSUPPORTED) rc = enqueue_attention(p);
     if (rc) return rc;
     return finish_launch("attention_gqa");
 }

@@ -39,6 +39,11 @@ struct AttnParams {
 };
 
 int enqueue_attention(const AttnParams &p);
+// Several query rows over a contiguous fp16 cache on the matrix cores;
+// UNSUPPORTED, before any launch, for what it does not take.
+int enqueue_attention_chunk(const AttnParams &p);
+// out = the merge of [row][split] partials, default q/out layout, D 64 or 128.
+void enqueue_attention_merge(const AttnParams &p, const float *part_o, const float *part_ml, int splits);
 // Upper bound of the split-partial bytes enqueue_attention needs for B
 // sequences of Hq heads, Sq query rows, head size D and `keys` cached keys.
 size_t attention_scratch_bytes(int B, int Hq, int Sq, int D, int keys);
