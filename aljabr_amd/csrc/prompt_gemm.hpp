@@ -18,9 +18,8 @@
 // What bounds it: the matrix cores (32 cycles per product of a 32x32x16
 // step, one to three products per weight), beside which one wave per SIMD
 // issues 16 FMAs per tile and scale group and the decode. NF4 MLP
-// 4096 x 14336: 512 tokens 725 -> 486 us, 2048 tokens 1.5 ms (0.96 PFLOP/s of
-// products); Q8_0 Q/K/V 3840 x 2560, 197 tokens 727 -> 33 us; Q4_K_M FFN
-// 4096 x 14336, 2048 tokens 5.24 -> 1.44 ms.
+// 4096 x 14336: 512 tokens 742 -> 452 us; Q8_0 Q/K/V 3840 x 2560, 197 tokens
+// 727 -> 32 us; Q4_K_M FFN 4096 x 14336, 2048 tokens 5.35 -> 1.45 ms.
 //
 // Arithmetic, as in the small-M kernels: weights are exact fp16 integers (or
 // NF4's exact H + R level pair, or Q6_K's two exact parts), the block scales
