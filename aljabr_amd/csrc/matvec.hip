@@ -495,8 +495,10 @@ int enqueue_matmul_nf4(float *C, const float *A, const uint8_t *Bq, const float 
     // Prompts (without a session's own buffer): the weights once for all
     // tokens instead of once per 64.
     if (!part && bs == 64 && aligned(Bq, 16) && prompt_nf4(M, N, K)) {
+        // One part where the passes round the activations (nf4_gemm_kernel takes the call).
         const RowsOut o{C, Bq, absmax, N};
-        const int rc = enqueue_prompt_gemm(&o, 1, A, K, ALJABR_ROCM_TYPE_NF4, K % 1024 == 0 ? 1 : 2, M);
+        const int rc = enqueue_prompt_gemm(&o, 1, A, K, ALJABR_ROCM_TYPE_NF4,
+                                           K % 1024 == 0 && aligned(absmax, 8) ? 1 : 2, M);
         if (rc != ALJABR_ROCM_ERR_UNSUPPORTED) return rc;
     }
     // M >= 2 on the matrix cores when the shape allows (deterministic;

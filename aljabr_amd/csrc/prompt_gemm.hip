@@ -129,6 +129,19 @@ Plan make_plan(int f, int xp, int M, int N, int chunks, int cus) {
     return best;
 }
 
+// Whether the passes that the call replaces run any of its tokens in fp32:
+// shapes and alignments that the matrix-core passes do not take, and the last
+// single token left by the GGUF passes of 8 or 32. Those tokens keep fp32's
+// range and relative accuracy, so the rows are scaled (unscaled, an element
+// past 65504 is infinite and one under 2^-14 loses its last bits).
+bool fp32_passes(const RowsOut *outs, int nseg, int f, int K, int M) {
+    bool aligned_all = true;
+    for (int i = 0; i < nseg; ++i)
+        aligned_all = aligned_all && (f == kPgNF4 ? aligned(outs[i].absmax, 8) : aligned(outs[i].w, 16));
+    if (!aligned_all || K % (f == kPgNF4 ? 256 : 512) != 0) return true;
+    return f == kPgNF4 ? false : M % (f == kPgQ40 || f == kPgQ80 ? 8 : 32) == 1;
+}
+
 }  // namespace
 
 int enqueue_prompt_gemm(const RowsOut *outs, int nseg, const float *A, int K, int type, int xparts, int M) {
@@ -155,9 +168,7 @@ int enqueue_prompt_gemm(const RowsOut *outs, int nseg, const float *A, int K, in
         a.absmax[i] = o.absmax;
         a.end[i] = static_cast<int>(end);
     }
-    // Shapes whose passes compute in fp32 (they are not the matrix-core
-    // kernels') keep fp32's range: their rows are scaled.
-    const bool scaled = xparts == 2 && K % (f == kPgNF4 ? 256 : 512) != 0;
+    const bool scaled = xparts == 2 && fp32_passes(outs, nseg, f, K, M);
     a.nseg = nseg;
     a.N = static_cast<int>(end);
     a.K = K;

@@ -81,3 +81,49 @@ def test_stacked_prompt(rocm, dev, oracle, t, ns, k, m):
     for got, again, raw, n in zip(*outs, raws, ns):
         assert np.array_equal(got, again)
         assert rel_l2(got, x.astype(np.float64) @ _decoded(oracle, t, raw, n, k).T) <= TOL
+
+
+def _put_at(dev, a, offset):
+    """The bytes of `a` on the device, `offset` bytes past an aligned address."""
+    import torch
+    raw = np.ascontiguousarray(a).view(np.uint8).ravel()
+    t = dev.empty(raw.size + offset, np.uint8)
+    t[offset:] = torch.from_numpy(raw).to(t.device)
+    torch.cuda.synchronize()
+    return t, t.data_ptr() + offset
+
+
+# Tokens that the passes run in fp32: weights off 16-byte alignment (4, 8), and
+# the last single token of the passes of 8 (Q4_0, Q8_0) and 32 (K-quants).
+# Elements past fp16's range and rows far below it keep their accuracy.
+@pytest.mark.parametrize("t,n,k,m,offset,row", [
+    (Q4_0, 96, 1024, 130, 4, 3), (Q8_0, 96, 512, 130, 8, 3), (Q4_0, 64, 1024, 129, 0, 128), (Q8_0, 96, 512, 193, 0, 192),
+    (Q6_K, 300, 1024, 129, 0, 128), (Q4_K, 300, 1024, 193, 0, 192)])
+@pytest.mark.parametrize("size", [1e5, 1e-5])
+def test_gguf_prompt_keeps_fp32_range(rocm, dev, oracle, t, n, k, m, offset, row, size):
+    raw = _weights(oracle, t, n, k, 3)
+    x = oracle.normal(4, m * k).reshape(m, k)
+    x[row] *= size
+    w, wp = _put_at(dev, raw, offset)
+    y, xd = dev.empty(m * n), dev.put(x)
+    rocm.call("aljabr_rocm_matvec_tb_batch", dev.ptr(y), dev.ptr(xd), wp, k, n, t, m)
+    got = dev.get(y).reshape(m, n)
+    ref = x.astype(np.float64) @ _decoded(oracle, t, raw, n, k).T
+    for i in range(m):
+        assert rel_l2(got[i], ref[i]) <= TOL, i
+
+
+@pytest.mark.parametrize("n,k,m", [(96, 1280, 130), (96, 1024, 130)])
+@pytest.mark.parametrize("size", [1e5, 1e-5])
+def test_nf4_prompt_with_absmax_off_8_bytes(rocm, dev, oracle, n, k, m, size):
+    """The passes run these in fp32, whatever K: no rounding, fp32's range."""
+    codes, absmax = oracle.nf4_quantize(oracle.normal(5, n * k, 0.0, 0.02), 64)
+    x = oracle.normal(6, m * k).reshape(m, k)
+    x[3] *= size
+    a, ap = _put_at(dev, absmax, 4)
+    y, c, xd = dev.empty(m * n), dev.put(codes), dev.put(x)
+    rocm.call("aljabr_rocm_matvec_tb_batch_nf4", dev.ptr(y), dev.ptr(xd), dev.ptr(c), ap, k, n, 64, m)
+    got = dev.get(y).reshape(m, n)
+    ref = x.astype(np.float64) @ oracle.nf4_dequant(codes, absmax, n * k, 64).reshape(n, k).astype(np.float64).T
+    for i in range(m):
+        assert rel_l2(got[i], ref[i]) <= TOL, i
