@@ -168,7 +168,10 @@ int enqueue_prompt_gemm(const RowsOut *outs, int nseg, const float *A, int K, in
         a.absmax[i] = o.absmax;
         a.end[i] = static_cast<int>(end);
     }
-    const bool scaled = xparts == 2 && fp32_passes(outs, nseg, f, K, M);
+    // Q4_K's rows always are: a sub-block's sum of 32 activations leaves fp16's
+    // range before they do, and its parts would be inf - inf. Scaled it is
+    // below 2^14.
+    const bool scaled = f == kPgQ4K || (xparts == 2 && fp32_passes(outs, nseg, f, K, M));
     a.nseg = nseg;
     a.N = static_cast<int>(end);
     a.K = K;

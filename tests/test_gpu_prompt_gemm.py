@@ -127,3 +127,19 @@ def test_nf4_prompt_with_absmax_off_8_bytes(rocm, dev, oracle, n, k, m, size):
     ref = x.astype(np.float64) @ oracle.nf4_dequant(codes, absmax, n * k, 64).reshape(n, k).astype(np.float64).T
     for i in range(m):
         assert rel_l2(got[i], ref[i]) <= TOL, i
+
+
+@pytest.mark.parametrize("n,k", [(12300, 4096), (300, 1024), (300, 1280)])
+@pytest.mark.parametrize("size", [3e3, 6e4])
+def test_q4_k_prompt_one_signed_rows(rocm, dev, oracle, n, k, size):
+    """A sub-block's 32 activations are each in fp16's range, their sum is not."""
+    m = 130
+    raw = _weights(oracle, Q4_K, n, k, 3)
+    x = oracle.normal(4, m * k).reshape(m, k)
+    x[5] = size + x[5]
+    y, w, xd = dev.empty(m * n), dev.put(raw), dev.put(x)
+    rocm.call("aljabr_rocm_matvec_tb_batch", dev.ptr(y), dev.ptr(xd), dev.ptr(w), k, n, Q4_K, m)
+    got = dev.get(y).reshape(m, n)
+    ref = _parts(x, n > 8192) @ _decoded(oracle, Q4_K, raw, n, k).T
+    for i in range(m):
+        assert rel_l2(got[i], ref[i]) <= TOL, i
