@@ -65,7 +65,8 @@ int enqueue_matmul_multi(float *const *C, const float *A, const uint8_t *const *
     if (same && prompt_gguf(type[0], batch, N[0], K)) {
         RowsOut outs[3];
         const int xparts = prompt_xparts(type[0], N[0], K);
-        bool stack = true;                       // one precision for the stack
+        // One precision for the stack, and no last token beside it.
+        bool stack = prompt_last_token(xparts, batch) == 0;
         for (int i = 0; i < n; ++i) {
             outs[i] = RowsOut{C[i], B[i], nullptr, N[i]};
             stack = stack && prompt_gguf(type[0], batch, N[i], K) && prompt_xparts(type[0], N[i], K) == xparts;

@@ -239,6 +239,9 @@ bool q4k_rounds_activations(int N, int K);
 // GEMM takes (those of the passes it replaces).
 bool prompt_gguf(int type, int M, int N, int K);
 int prompt_xparts(int type, int N, int K);
+// Tokens of a GGUF prompt with rounded activations that run on the batch-1
+// kernel instead: the single one that the passes of 32 leave over, in fp32.
+int prompt_last_token(int xparts, int M);
 // GGUF Q4_0 / Q8_0 GEMM pass of M <= 16 tokens with the activations held in
 // registers (K % 2048 == 0, A 16-byte aligned; up to three stacked matrices
 // of one type, all but the last a multiple of 16 rows; fp32-accurate,

@@ -521,11 +521,19 @@ int prompt_xparts(int type, int N, int K) {
     return type == ALJABR_ROCM_TYPE_Q4_K && q4k_rounds_activations(N, K) ? 1 : 2;
 }
 
+int prompt_last_token(int xparts, int M) { return xparts == 1 && M % 32 == 1 ? 1 : 0; }
+
 int enqueue_matmul_gguf(float *C, const float *A, const uint8_t *B, int K, int N, int type, int M, float *part,
                         size_t part_floats) {
-    if (!part && prompt_gguf(type, M, N, K)) {
+    const int xparts = prompt_xparts(type, N, K);
+    const int last = prompt_last_token(xparts, M);
+    if (!part && prompt_gguf(type, M - last, N, K)) {
         const RowsOut o{C, B, nullptr, N};
-        const int rc = enqueue_prompt_gemm(&o, 1, A, K, type, prompt_xparts(type, N, K), M);
+        const int rc = enqueue_prompt_gemm(&o, 1, A, K, type, xparts, M - last);
+        if (rc == ALJABR_ROCM_OK && last) {
+            const size_t m0 = static_cast<size_t>(M - 1);
+            return enqueue_matmul_gguf(C + m0 * N, A + m0 * K, B, K, N, type, 1, nullptr, 0);
+        }
         if (rc != ALJABR_ROCM_ERR_UNSUPPORTED) return rc;
     }
     if (type == ALJABR_ROCM_TYPE_Q4_K || type == ALJABR_ROCM_TYPE_Q6_K)

@@ -143,3 +143,32 @@ def test_q4_k_prompt_one_signed_rows(rocm, dev, oracle, n, k, size):
     ref = _parts(x, n > 8192) @ _decoded(oracle, Q4_K, raw, n, k).T
     for i in range(m):
         assert rel_l2(got[i], ref[i]) <= TOL, i
+
+
+@pytest.mark.parametrize("m", [65, 97, 129])
+def test_last_q4_k_token_is_not_rounded(rocm, dev, oracle, m):
+    """Where the passes round a Q4_K matrix's activations, a single token left
+    over runs on the batch-1 kernel, in fp32."""
+    n, k = 12300, 4096
+    raw = _weights(oracle, Q4_K, n, k, 3)
+    x = oracle.normal(4, m * k).reshape(m, k)
+    x[-1] *= 1e5
+    y, w, xd = dev.empty(m * n), dev.put(raw), dev.put(x)
+    rocm.call("aljabr_rocm_matvec_tb_batch", dev.ptr(y), dev.ptr(xd), dev.ptr(w), k, n, Q4_K, m)
+    got = dev.get(y).reshape(m, n)
+    w64 = _decoded(oracle, Q4_K, raw, n, k)
+    assert rel_l2(got[-1], x[-1].astype(np.float64) @ w64.T) <= TOL
+    assert rel_l2(got[:-1], _parts(x[:-1], True) @ w64.T) <= TOL
+
+
+def test_last_q4_k_token_of_a_stack_is_not_rounded(rocm, dev, oracle):
+    ns, k, m = (12320, 12300, 64), 4096, 97
+    raws = [_weights(oracle, Q4_K, n, k, 3 + i) for i, n in enumerate(ns)]
+    x = oracle.normal(4, m * k).reshape(m, k)
+    ys, ws, xd = [dev.empty(m * n) for n in ns], [dev.put(r) for r in raws], dev.put(x)
+    rocm.call("aljabr_rocm_matvec_tb_triple_batch", *[dev.ptr(y) for y in ys], dev.ptr(xd), *[dev.ptr(w) for w in ws], k,
+              *ns, Q4_K, Q4_K, Q4_K, m)
+    for y, raw, n in zip(ys, raws, ns):
+        got, w64 = dev.get(y).reshape(m, n), _decoded(oracle, Q4_K, raw, n, k)
+        assert rel_l2(got[-1], x[-1].astype(np.float64) @ w64.T) <= TOL
+        assert rel_l2(got[:-1], _parts(x[:-1], n > 8192) @ w64.T) <= TOL
