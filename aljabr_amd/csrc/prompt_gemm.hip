@@ -160,7 +160,9 @@ int enqueue_prompt_gemm(const RowsOut *outs, int nseg, const float *A, int K, in
         a.end[i] = 0x7fffffff;
         if (i >= nseg) continue;
         const RowsOut &o = outs[i];
-        const size_t wa = f == kPgNF4 || f == kPgQ4K ? 16 : 4;
+        // NF4 codes are read 16 bytes at a time; the K-quants' callers refuse
+        // weights off 16 bytes at every batch size.
+        const size_t wa = f == kPgQ40 || f == kPgQ80 ? 4 : 16;
         if (o.n <= 0 || !aligned(o.w, wa) || (i < nseg - 1 && o.n % 32 != 0)) return ALJABR_ROCM_ERR_UNSUPPORTED;
         end += o.n;
         if (end > 0x7fff0000LL) return ALJABR_ROCM_ERR_UNSUPPORTED;

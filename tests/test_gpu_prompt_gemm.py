@@ -172,3 +172,15 @@ def test_last_q4_k_token_of_a_stack_is_not_rounded(rocm, dev, oracle):
         got, w64 = dev.get(y).reshape(m, n), _decoded(oracle, Q4_K, raw, n, k)
         assert rel_l2(got[-1], x[-1].astype(np.float64) @ w64.T) <= TOL
         assert rel_l2(got[:-1], _parts(x[:-1], n > 8192) @ w64.T) <= TOL
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q6_K])
+@pytest.mark.parametrize("m", [8, 130])
+def test_k_quants_need_16_byte_weights(rocm, dev, oracle, t, m):
+    """Refused at every batch size, as the entry point says."""
+    n, k = 64, 512
+    w, wp = _put_at(dev, _weights(oracle, t, n, k, 3), 4)
+    y, xd = dev.empty(m * n), dev.put(oracle.normal(4, m * k))
+    with pytest.raises(rocm.RocmError) as e:
+        rocm.call("aljabr_rocm_matvec_tb_batch", dev.ptr(y), dev.ptr(xd), wp, k, n, t, m)
+    assert e.value.status == rocm.ERR_BAD_ARGUMENT
