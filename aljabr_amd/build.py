@@ -30,12 +30,16 @@ HIPCC = os.environ.get("HIPCC") or shutil.which("hipcc") or "/opt/rocm/bin/hipcc
 # the argument buffer; the compiler also emits the fallback that reads them.
 DEVICE_FLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-mllvm",
                 "-amdgpu-kernarg-preload-count=14"]
+# The prompt GEMM runs one wave per SIMD. There the compiler would put the
+# matrix products in AGPRs, which the vector ALU cannot read without a copy of
+# each (Q4_K_M FFN, 2048 tokens: 2.13 ms so, 1.48 ms with them in VGPRs).
+FILE_FLAGS = {f"prompt_{t}.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"] for t in ("nf4", "q40", "q80", "q4k", "q6k")}
 COMMON = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-Wall", "-Wno-unused-function"]
 
 
 def _compile(src: str) -> str:
     obj = os.path.join(BUILD, os.path.basename(src) + ".o")
-    cmd = [HIPCC, *COMMON, *DEVICE_FLAGS, "-c", src, "-o", obj]
+    cmd = [HIPCC, *COMMON, *DEVICE_FLAGS, *FILE_FLAGS.get(os.path.basename(src), []), "-c", src, "-o", obj]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src}:\n{res.stderr}")

@@ -18,7 +18,7 @@ using pg::half8;
 // of 8 sub-blocks.
 __global__ __launch_bounds__(256) void prompt_pack_kernel(const float *x, u32x4 *xh, u32x4 *xl, _Float16 *sums, int M,
                                                           int K, int tiles, int nf4, const float *scale) {
-    __shared__ float part[4][64];
+    __shared__ double part[4][64];
     const int tid = threadIdx.x, lane = tid & 63, j = tid >> 6, h = lane >> 5, i = lane & 31;
     const int tile = blockIdx.x % tiles, kb = blockIdx.x / tiles;
     const int m = 32 * tile + i;
@@ -36,13 +36,13 @@ __global__ __launch_bounds__(256) void prompt_pack_kernel(const float *x, u32x4 
         for (int e = 0; e < 8; ++e) v[e] *= inv;
     }
     half8 hi, lo;
-    float t = 0.0f;
+    double t = 0.0;                              // the min term is several times the result: no rounding here
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         hi[e] = static_cast<_Float16>(v[e]);
         lo[e] = isinf(static_cast<float>(hi[e])) ? static_cast<_Float16>(0.0f)
                                                  : static_cast<_Float16>(v[e] - static_cast<float>(hi[e]));
-        t += xl ? v[e] : static_cast<float>(hi[e]);
+        t += static_cast<double>(xl ? v[e] : static_cast<float>(hi[e]));
     }
     const size_t at = (static_cast<size_t>(blockIdx.x) * 4 + j) * 64 + lane;
     xh[at] = __builtin_bit_cast(u32x4, hi);
@@ -52,12 +52,44 @@ __global__ __launch_bounds__(256) void prompt_pack_kernel(const float *x, u32x4 
     __syncthreads();
     if (tid < 64) {
         const int sb = tid >> 5;                     // sub-block of the chunk: steps 2sb and 2sb + 1
-        const float s = (part[2 * sb][i] + part[2 * sb][32 + i]) + (part[2 * sb + 1][i] + part[2 * sb + 1][32 + i]);
-        const _Float16 sh = static_cast<_Float16>(s);
+        const double s = (part[2 * sb][i] + part[2 * sb][32 + i]) + (part[2 * sb + 1][i] + part[2 * sb + 1][32 + i]);
+        const _Float16 sh = static_cast<_Float16>(static_cast<float>(s));
         _Float16 *dst = sums + ((static_cast<size_t>(kb >> 2) * tiles + tile) * 64 + i) * 8 + 2 * (kb & 3) + sb;
         dst[0] = sh;
-        dst[32 * 8] = static_cast<_Float16>(s - static_cast<float>(sh));
+        dst[32 * 8] = static_cast<_Float16>(static_cast<float>(s - static_cast<double>(sh)));
     }
+}
+
+// Y = the K slices' partial sums, added in double: up to 32 of them would add
+// as many roundings to the result as the slices save. Loads in flight as in
+// slice_sum (device.hpp).
+template <int U>
+__device__ __forceinline__ double slice_sum_f64(const float *p, size_t stride, int slices) {
+    double acc = 0.0;
+    for (int s0 = 0; s0 < slices; s0 += U) {
+        float v[U];
+#pragma unroll
+        for (int j = 0; j < U; ++j) v[j] = p[static_cast<size_t>(min(s0 + j, slices - 1)) * stride];
+#pragma unroll
+        for (int j = 0; j < U; ++j)
+            if (s0 + j < slices) acc += static_cast<double>(v[j]);
+    }
+    return acc;
+}
+
+__global__ __launch_bounds__(256) void prompt_sum_kernel(PgArgs a) {
+    const int n = blockIdx.x * 256 + threadIdx.x, m = blockIdx.y;
+    if (n >= a.N) return;
+    const float *p = a.part + static_cast<size_t>(m) * a.N + n;
+    const size_t stride = static_cast<size_t>(a.M) * a.N;
+    const double v = a.slices <= 4   ? slice_sum_f64<4>(p, stride, a.slices)
+                     : a.slices <= 8 ? slice_sum_f64<8>(p, stride, a.slices)
+                                     : slice_sum_f64<16>(p, stride, a.slices);
+    int s = (n >= a.end[0]) + (n >= a.end[1]);
+    if (s > a.nseg - 1) s = a.nseg - 1;
+    const int start = s == 0 ? 0 : s == 1 ? a.end[0] : a.end[1];
+    const int rows = (s == 0 ? a.end[0] : s == 1 ? a.end[1] : a.end[2]) - start;
+    (s == 0 ? a.y[0] : s == 1 ? a.y[1] : a.y[2])[static_cast<size_t>(m) * rows + (n - start)] = static_cast<float>(v);
 }
 
 // The plan's constants are fits of a sweep over tiles, slices and formats
@@ -70,11 +102,20 @@ constexpr float kPartialMb = 128.0f;                  // bounds the K slices' pa
 // [2^8, 2^9): with it any fp32 row fits the fp16 parts. One workgroup a row.
 __global__ __launch_bounds__(256) void prompt_scale_kernel(const float *x, float *scale, int K) {
     __shared__ float best[4];
-    const float *row = x + static_cast<size_t>(blockIdx.x) * K;
+    const float4 *row = reinterpret_cast<const float4 *>(x + static_cast<size_t>(blockIdx.x) * K);
+    const int quads = K >> 2;                            // K % 32 == 0
     float top = 0.0f;
-    for (int k = threadIdx.x; k < K; k += 256) {
-        const float v = fabsf(row[k]);
-        if (v <= 3.4028235e38f) top = fmaxf(top, v);
+    for (int k0 = threadIdx.x; k0 < quads; k0 += 4 * 256) {
+        float4 v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = k0 + 256 * i < quads ? row[k0 + 256 * i] : float4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float e[4] = {fabsf(v[i].x), fabsf(v[i].y), fabsf(v[i].z), fabsf(v[i].w)};
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (e[j] <= 3.4028235e38f) top = fmaxf(top, e[j]);
+        }
     }
     top = wave_max(top);
     if ((threadIdx.x & 63) == 0) best[threadIdx.x >> 6] = top;
@@ -234,10 +275,9 @@ int enqueue_prompt_gemm(const RowsOut *outs, int nseg, const float *A, int K, in
             }
             if (rc != ALJABR_ROCM_OK) return rc;
         }
-        if (a.part) {
-            const int rc = enqueue_slice_sum(a.y, a.end, nseg, mm, a.N, a.part, p.slices, false);
-            if (rc != ALJABR_ROCM_OK) return rc;
-        }
+        if (a.part)
+            hipLaunchKernelGGL(prompt_sum_kernel, dim3(static_cast<unsigned>((a.N + 255) / 256), static_cast<unsigned>(mm)),
+                               dim3(256), 0, s, a);
     }
     return ALJABR_ROCM_OK;
 }

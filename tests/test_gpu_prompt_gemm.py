@@ -184,3 +184,45 @@ def test_k_quants_need_16_byte_weights(rocm, dev, oracle, t, m):
     with pytest.raises(rocm.RocmError) as e:
         rocm.call("aljabr_rocm_matvec_tb_batch", dev.ptr(y), dev.ptr(xd), wp, k, n, t, m)
     assert e.value.status == rocm.ERR_BAD_ARGUMENT
+
+
+def _random_blocks(t, n, k, seed):
+    """Random Q4_0 / Q8_0 rows, made quickly."""
+    g = np.random.default_rng(seed)
+    b = np.empty((n * k // 32, 18 if t == Q4_0 else 34), np.uint8)
+    b[:, 2:] = g.integers(0, 256, (b.shape[0], b.shape[1] - 2), np.uint8)
+    b[:, :2] = (g.random(b.shape[0], np.float32) * (0.1 if t == Q4_0 else 0.01)).astype(np.float16).view(np.uint8).reshape(-1, 2)
+    return b.reshape(n, -1)
+
+
+@pytest.mark.parametrize("t,n,k,m", [(Q8_0, 4096, 14336, 512), (Q4_0, 4096, 14336, 512), (Q8_0, 2816, 1024, 1000),
+                                     (Q8_0, 1024, 1024, 40), (Q4_0, 256, 14336, 64)])
+def test_long_sums_keep_their_accuracy(rocm, dev, oracle, t, n, k, m):
+    """The fp32 sums over K round no more than those of the passes of 8 tokens.
+    A product's own rounding is 0.75e-7 and a chain of L additions adds 2.5e-8
+    sqrt(L / 2): the passes' chains (of 8 to 16 blocks, then 8 waves or the
+    slices) measure 0.97e-7 at K = 1024 and 1.19e-7 at K = 14336, one chain
+    over all of K 1.25e-7 and 2.08e-7."""
+    raw = _random_blocks(t, n, k, 3)
+    x = oracle.normal(4, m * k).reshape(m, k)
+    y, w, xd = dev.empty(m * n), dev.put(raw), dev.put(x)
+    rocm.call("aljabr_rocm_matvec_tb_batch", dev.ptr(y), dev.ptr(xd), dev.ptr(w), k, n, t, m)
+    step = 31 if n > 1024 else 3
+    got = dev.get(y).reshape(m, n)[:, ::step]
+    raw = np.ascontiguousarray(raw[::step])
+    ref = x.astype(np.float64) @ _decoded(oracle, t, raw.ravel(), len(raw), k).T
+    assert rel_l2(got, ref) <= (1.0e-7 if k == 1024 else 1.19e-7)
+
+
+def test_q4_k_prompt_is_no_further_off_than_fp32(rocm, dev, oracle):
+    """K % 512 != 0: the vector kernel's fp32 gives 1.13e-7 here; sub-block sums
+    rounded to fp32 before their split gave 1.30e-7."""
+    n, k, m = 2304, 2304, 512
+    raw = _weights(oracle, Q4_K, n, k, 3)
+    x = oracle.normal(4, m * k).reshape(m, k)
+    y, w, xd = dev.empty(m * n), dev.put(raw), dev.put(x)
+    vec = dev.empty(8 * n)
+    rocm.call("aljabr_rocm_matvec_tb_batch", dev.ptr(y), dev.ptr(xd), dev.ptr(w), k, n, Q4_K, m)
+    rocm.call("aljabr_rocm_matvec_tb_batch", dev.ptr(vec), dev.ptr(xd), dev.ptr(w), k, n, Q4_K, 8)
+    ref = x.astype(np.float64) @ _decoded(oracle, Q4_K, raw, n, k).T
+    assert rel_l2(dev.get(y).reshape(m, n), ref) <= rel_l2(dev.get(vec).reshape(8, n), ref[:8])
