@@ -92,12 +92,6 @@ __global__ __launch_bounds__(256) void prompt_sum_kernel(PgArgs a) {
     (s == 0 ? a.y[0] : s == 1 ? a.y[1] : a.y[2])[static_cast<size_t>(m) * rows + (n - start)] = static_cast<float>(v);
 }
 
-// The plan's constants are fits of a sweep over tiles, slices and formats
-// (4096 x 14336 and 2560-wide layers, 64 to 2048 tokens): a chunk of four
-// token tiles took 1.65 us for two products (NF4, Q8_0), 2.4 us for Q6_K's
-// three; the slice sum moves ~5 TB/s.
-constexpr int kPassTokens = 4096;                    // bounds the activation image
-constexpr float kPartialMb = 128.0f;                  // bounds the K slices' partial sums
 // The power of two that brings a token row's largest finite magnitude into
 // [2^8, 2^9): with it any fp32 row fits the fp16 parts. One workgroup a row.
 __global__ __launch_bounds__(256) void prompt_scale_kernel(const float *x, float *scale, int K) {
@@ -127,7 +121,19 @@ __global__ __launch_bounds__(256) void prompt_scale_kernel(const float *x, float
     scale[blockIdx.x] = ldexpf(1.0f, (e < -100 ? -100 : e) - 9);
 }
 
+// What a call holds of the stream's scratch: the activation image of a pass of
+// tokens, the weight image of a panel of rows, the K slices' partial sums over
+// all panels.
+constexpr int kPassTokens = 4096;
+constexpr size_t kImageBytes = size_t{512} << 20;     // bounds the activation image
 constexpr size_t kPanelBytes = size_t{128} << 20;     // bounds the weight image
+constexpr float kPartialMb = 128.0f;                  // bounds the K slices' partial sums
+constexpr size_t kMaxScratch = size_t{1} << 30;       // a call past it keeps the passes (K past 10^6)
+
+// The plan's constants are fits of a sweep over tiles, slices and formats
+// (4096 x 14336 and 2560-wide layers, 64 to 2048 tokens): a chunk of four
+// token tiles took 1.65 us for two products (NF4, Q8_0), 2.4 us for Q6_K's
+// three; the slice sum moves ~5 TB/s.
 constexpr float kFixedUs = 3.0f, kReduceUs = 3.0f, kMbPerUs = 5.0f;
 
 // Tiles of 32 tokens per wave (2 or 4) and K slices for M tokens over N
@@ -136,11 +142,12 @@ constexpr float kFixedUs = 3.0f, kReduceUs = 3.0f, kMbPerUs = 5.0f;
 //
 // K slices trade idle CUs and ragged last rounds against the partial sums'
 // traffic: the least of rounds * (chunks * chunk time + fixed) + slice sum.
+// N is the rows of one panel, `all` those whose partial sums are held.
 struct Plan {
     int mt, mt_groups, n_groups, per, slices;
 };
 
-Plan make_plan(int f, int xp, int M, int N, int chunks, int cus) {
+Plan make_plan(int f, int xp, int M, int N, int all, int chunks, int cus) {
     const int quantum = f == kPgQ4K || f == kPgQ6K ? 4 : 1;
     // Microseconds of a workgroup's chunk: 32 cycles per product and its share
     // of the decode and the scaling.
@@ -148,12 +155,13 @@ Plan make_plan(int f, int xp, int M, int N, int chunks, int cus) {
     Plan best{};
     float best_us = 0.0f;
     const float out_mb = 4e-6f * static_cast<float>(M) * static_cast<float>(N);
+    const float held_mb = 4e-6f * static_cast<float>(M) * static_cast<float>(all);
     const int n_groups = (N + 64 * kPgWaves - 1) / (64 * kPgWaves);
     for (int mt = 4; mt >= 2; mt -= 2) {
         const float chunk_us = (0.4f + 0.68f * products) * (mt == 4 ? 1.0f : 0.55f);
         const int mt_groups = (M + 32 * mt - 1) / (32 * mt);
         for (int s = 1; s <= 32; ++s) {
-            if (s > 1 && (s * out_mb > kPartialMb || chunks / s < quantum)) break;
+            if (s > 1 && (s * held_mb > kPartialMb || chunks / s < quantum)) break;
             Plan p{mt, mt_groups, n_groups, 0, 0};
             p.per = (chunks + s - 1) / s;
             p.per = (p.per + quantum - 1) / quantum * quantum;
@@ -228,22 +236,39 @@ int enqueue_prompt_gemm(const RowsOut *outs, int nseg, const float *A, int K, in
     const int all_tiles = (a.N + 31) / 32;
     const int panels = static_cast<int>((all_tiles * (tile_codes + tile_aux) + kPanelBytes - 1) / kPanelBytes);
     const int panel = (all_tiles + panels - 1) / panels;
-    for (int m0 = 0; m0 < M; m0 += kPassTokens) {
-        const int mm = std::min(M - m0, kPassTokens);
-        const Plan p = make_plan(f, xparts, mm, std::min(panel * 32, a.N), a.chunks, cus);
+    const size_t image = (panel * (tile_codes + tile_aux) + 255) & ~size_t{255};
+    const size_t fit = kImageBytes / (static_cast<size_t>(xparts) * a.chunks * 128) / 128 * 128;
+    const int pass = static_cast<int>(std::min(static_cast<size_t>(kPassTokens), std::max(fit, size_t{128})));
+    // Bytes of a pass: its planes, sub-block sums, row scales and partial sums.
+    struct Layout {
+        size_t plane, sums, scales, parts;
+    };
+    const auto layout = [&](const Plan &p, int mm) {
+        const size_t tiles = static_cast<size_t>(p.mt_groups) * p.mt;
+        return Layout{a.chunks * tiles * 4096, f == kPgQ4K ? (a.chunks / 4) * tiles * 1024 : 0,
+                      scaled ? (static_cast<size_t>(mm) * sizeof(float) + 255) & ~size_t{255} : 0,
+                      p.slices > 1 ? static_cast<size_t>(p.slices) * mm * a.N * sizeof(float) : 0};
+    };
+    const auto plan = [&](int mm) { return make_plan(f, xparts, mm, std::min(panel * 32, a.N), a.N, a.chunks, cus); };
+    // One buffer for all passes, before any launch: a whole pass's and the
+    // last one's, whose plan may take more slices.
+    size_t bytes = 0;
+    for (const int mm : {std::min(M, pass), (M - 1) % pass + 1}) {
+        const Layout l = layout(plan(mm), mm);
+        bytes = std::max(bytes, xparts * l.plane + l.sums + image + l.scales + l.parts);
+    }
+    if (bytes > kMaxScratch) return ALJABR_ROCM_ERR_UNSUPPORTED;
+    uint8_t *buf = static_cast<uint8_t *>(stream_scratch_try(bytes, kScratchPartials));
+    if (!buf) return ALJABR_ROCM_ERR_UNSUPPORTED;
+    for (int m0 = 0; m0 < M; m0 += pass) {
+        const int mm = std::min(M - m0, pass);
+        const Plan p = plan(mm);
+        const auto [plane, sums, scales, parts] = layout(p, mm);
         a.M = mm;
         a.per = p.per;
         a.slices = p.slices;
         a.mt_groups = p.mt_groups;
         a.tiles = p.mt_groups * p.mt;
-        const size_t plane = static_cast<size_t>(a.chunks) * a.tiles * 4096;
-        const size_t sums = f == kPgQ4K ? static_cast<size_t>(a.chunks / 4) * a.tiles * 1024 : 0;
-        const size_t image = (panel * (tile_codes + tile_aux) + 255) & ~size_t{255};
-        const size_t scales = scaled ? (static_cast<size_t>(mm) * sizeof(float) + 255) & ~size_t{255} : 0;
-        const size_t parts = p.slices > 1 ? static_cast<size_t>(p.slices) * mm * a.N * sizeof(float) : 0;
-        uint8_t *buf =
-            static_cast<uint8_t *>(stream_scratch_try(xparts * plane + sums + image + scales + parts, kScratchPartials));
-        if (!buf) return m0 == 0 ? ALJABR_ROCM_ERR_UNSUPPORTED : ALJABR_ROCM_ERR_BUFFER;
         uint8_t *xl = xparts == 2 ? buf + plane : nullptr;
         uint8_t *next = buf + xparts * plane;
         a.xh = buf;

@@ -226,3 +226,83 @@ def test_q4_k_prompt_is_no_further_off_than_fp32(rocm, dev, oracle):
     rocm.call("aljabr_rocm_matvec_tb_batch", dev.ptr(vec), dev.ptr(xd), dev.ptr(w), k, n, Q4_K, 8)
     ref = x.astype(np.float64) @ _decoded(oracle, Q4_K, raw, n, k).T
     assert rel_l2(dev.get(y).reshape(m, n), ref) <= rel_l2(dev.get(vec).reshape(8, n), ref[:8])
+
+
+def _fresh_thread(fn):
+    """fn on a thread, and so a stream, of its own: no scratch held before."""
+    import threading
+    out = []
+
+    def body():
+        try:
+            out.append(fn())
+        except BaseException as e:               # re-raised on the test's thread
+            out.append(e)
+
+    t = threading.Thread(target=body)
+    t.start()
+    t.join(timeout=100)
+    assert not t.is_alive(), "worker thread did not finish"
+    if isinstance(out[0], BaseException):
+        raise out[0]
+    return out[0]
+
+
+def _held(rocm):
+    import ctypes
+    n = ctypes.c_size_t(0)
+    rocm.call("aljabr_rocm_stream_scratch_bytes", ctypes.byref(n))
+    return n.value
+
+
+def test_scratch_is_bounded_over_all_panels(rocm, dev):
+    """The K slices' partial sums of all weight panels together keep to their bound."""
+    import torch
+    n, k, m = 152064, 8192, 384
+    w = torch.zeros(n * k // 256 * 210, dtype=torch.uint8, device="cuda:0")
+    x, y = torch.zeros(m * k, device="cuda:0"), torch.empty(m * n, device="cuda:0")
+    torch.cuda.synchronize()
+
+    def body():
+        rocm.call("aljabr_rocm_matvec_tb_batch", dev.ptr(y), dev.ptr(x), dev.ptr(w), k, n, Q6_K, m)
+        return _held(rocm)
+
+    assert 4 * m * k <= _fresh_thread(body) <= 512 << 20
+    assert not y.any()
+
+
+# More than one panel of the weight image (128 MiB), segments that end inside
+# a panel and one that crosses its end, with K slices (n small) and without.
+@pytest.mark.parametrize("t,ns,k,m", [(Q8_0, (8032, 6016, 1001), 14336, 40), (Q4_0, (59008, 4032, 1003), 4096, 600)])
+def test_prompt_panels(rocm, dev, oracle, t, ns, k, m):
+    raws = [_random_blocks(t, n, k, 30 + i) for i, n in enumerate(ns)]
+    x = oracle.normal(8, m * k).reshape(m, k)
+    ws, xd, ys = [dev.put(r) for r in raws], dev.put(x), [dev.empty(m * n) for n in ns]
+
+    def body():
+        rocm.call("aljabr_rocm_matvec_tb_triple_batch", *[dev.ptr(y) for y in ys], dev.ptr(xd),
+                  *[dev.ptr(w) for w in ws], k, *ns, t, t, t, m)
+        return _held(rocm)
+
+    assert _fresh_thread(body) >= (64 << 20) + 4 * m * k
+    g = np.random.default_rng(1)
+    for y, raw, n in zip(ys, raws, ns):
+        got = dev.get(y).reshape(m, n)
+        rows = np.unique(np.concatenate([np.arange(0, n, 257), np.arange(n - 40, n), g.integers(0, n, 64)]))
+        ref = x.astype(np.float64) @ _decoded(oracle, t, np.ascontiguousarray(raw[rows]).ravel(), len(rows), k).T
+        assert rel_l2(got[:, rows], ref) <= TOL
+        assert np.abs(got[:, rows] - ref).max() <= 20 * TOL * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("m", [4097, 4100, 8192 + 33])
+def test_prompt_token_passes(rocm, dev, oracle, m):
+    """More tokens than one pass of 4096 takes."""
+    n, k = 70, 512
+    raw = _weights(oracle, Q8_0, n, k, 3)
+    x = oracle.normal(4, m * k).reshape(m, k)
+    y, w, xd = dev.empty(m * n), dev.put(raw), dev.put(x)
+    rocm.call("aljabr_rocm_matvec_tb_batch", dev.ptr(y), dev.ptr(xd), dev.ptr(w), k, n, Q8_0, m)
+    got = dev.get(y).reshape(m, n)
+    ref = x.astype(np.float64) @ _decoded(oracle, Q8_0, raw, n, k).T
+    for i in range(m):
+        assert rel_l2(got[i], ref[i]) <= TOL, i
