@@ -6,6 +6,7 @@
 // one non-blocking stream per calling thread, explicit device buffers.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cstdarg>
 #include <cstring>
@@ -122,15 +123,22 @@ void *stream_scratch(size_t bytes, int slot) {
     Scratch &sc = c.scratch[s][slot];
     if (sc.bytes >= bytes) return sc.ptr;
     // Growing: the old buffer may still be read by queued work on this stream.
+    // By half of what was held (at most 256 MiB) if that is more: a prompt fed
+    // in chunks asks for a little more each time, and every growth waits here.
+    size_t want = std::max({bytes, size_t{1} << 20, sc.bytes + std::min(sc.bytes / 2, size_t{256} << 20)});
     if (sc.ptr) {
         (void)hipStreamSynchronize(s);
         (void)hipFree(sc.ptr);
         sc.ptr = nullptr;
         sc.bytes = 0;
     }
-    size_t want = bytes < (1u << 20) ? (1u << 20) : bytes;
     void *p = nullptr;
     hipError_t e = hipMalloc(&p, want);
+    if (e != hipSuccess && want > bytes) {
+        (void)hipGetLastError();                 // without the headroom
+        want = bytes;
+        e = hipMalloc(&p, want);
+    }
     if (e != hipSuccess) {
         hip_fail(e, ALJABR_ROCM_ERR_BUFFER, "scratch hipMalloc");
         return nullptr;

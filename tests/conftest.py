@@ -2,8 +2,10 @@
 on the CPU with no GPU calls."""
 from __future__ import annotations
 
+import ctypes
 import os
 import sys
+import threading
 
 import numpy as np
 import pytest
@@ -22,6 +24,33 @@ def rel_l2(actual, expected) -> float:
     e = np.asarray(expected, dtype=np.float64).ravel()
     den = np.linalg.norm(e)
     return float(np.linalg.norm(a - e) / (den if den > 0 else 1.0))
+
+
+def fresh_thread(fn):
+    """fn() on a thread, and so a library stream, of its own, which holds no
+    scratch before it; its result, or its exception raised here."""
+    out = []
+
+    def body():
+        try:
+            out.append((fn(), None))
+        except BaseException as e:               # re-raised on the test's thread
+            out.append((None, e))
+
+    t = threading.Thread(target=body)
+    t.start()
+    t.join(timeout=100)
+    assert not t.is_alive(), "worker thread did not finish"
+    if out[0][1] is not None:
+        raise out[0][1]
+    return out[0][0]
+
+
+def scratch_held(rocm) -> int:
+    """Bytes of scratch the library holds for the calling thread's stream."""
+    n = ctypes.c_size_t(0)
+    rocm.call("aljabr_rocm_stream_scratch_bytes", ctypes.byref(n))
+    return n.value
 
 
 @pytest.fixture(scope="session")

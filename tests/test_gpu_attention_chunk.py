@@ -9,7 +9,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
-from conftest import rel_l2
+from conftest import fresh_thread, rel_l2, scratch_held
 
 pytestmark = pytest.mark.gpu
 F16 = 1
@@ -74,3 +74,26 @@ def test_non_finite_rows_stay_apart(rocm, dev, b, sk, where, value):
     else:                                    # +inf scores give NaN, -inf ones leave the key out
         up = q[:, :, sq - 10:, 3] > 0
         assert np.isnan(got[:, :, sq - 10:][up]).all() and np.isfinite(got[:, :, sq - 10:][~up]).all()
+
+
+def test_growing_calls_rarely_reallocate(rocm, dev):
+    """A chunked prompt grows its keys with every call; the stream's scratch
+    grows geometrically, not with each (a growth waits for the stream)."""
+    import torch
+    hq, hkv, sq, d = 32, 8, 128, 128
+    q = torch.zeros(hq * sq * d, device="cuda:0")
+    out = torch.empty_like(q)
+    kv = torch.zeros(hkv * 8192 * d, dtype=torch.float16, device="cuda:0")
+    torch.cuda.synchronize()
+
+    def body():
+        seen = []
+        for sk in range(256, 8192 + 1, 128):
+            rocm.call("aljabr_rocm_attention_gqa", dev.ptr(out), dev.ptr(q), dev.ptr(kv), dev.ptr(kv), None, 1, hq, hkv,
+                      sq, sk, d, 1, 0.0, 1)
+            seen.append(scratch_held(rocm))
+        return seen
+
+    seen = fresh_thread(body)
+    assert seen[-1] >= 2 * 2 * hkv * 8192 * d
+    assert len(set(seen)) <= 16

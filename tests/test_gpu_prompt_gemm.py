@@ -12,7 +12,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
-from conftest import rel_l2
+from conftest import fresh_thread, rel_l2, scratch_held
 
 pytestmark = pytest.mark.gpu
 Q4_0, Q8_0, Q4_K, Q6_K = 2, 8, 12, 14
@@ -228,33 +228,6 @@ def test_q4_k_prompt_is_no_further_off_than_fp32(rocm, dev, oracle):
     assert rel_l2(dev.get(y).reshape(m, n), ref) <= rel_l2(dev.get(vec).reshape(8, n), ref[:8])
 
 
-def _fresh_thread(fn):
-    """fn on a thread, and so a stream, of its own: no scratch held before."""
-    import threading
-    out = []
-
-    def body():
-        try:
-            out.append(fn())
-        except BaseException as e:               # re-raised on the test's thread
-            out.append(e)
-
-    t = threading.Thread(target=body)
-    t.start()
-    t.join(timeout=100)
-    assert not t.is_alive(), "worker thread did not finish"
-    if isinstance(out[0], BaseException):
-        raise out[0]
-    return out[0]
-
-
-def _held(rocm):
-    import ctypes
-    n = ctypes.c_size_t(0)
-    rocm.call("aljabr_rocm_stream_scratch_bytes", ctypes.byref(n))
-    return n.value
-
-
 def test_scratch_is_bounded_over_all_panels(rocm, dev):
     """The K slices' partial sums of all weight panels together keep to their bound."""
     import torch
@@ -265,9 +238,9 @@ def test_scratch_is_bounded_over_all_panels(rocm, dev):
 
     def body():
         rocm.call("aljabr_rocm_matvec_tb_batch", dev.ptr(y), dev.ptr(x), dev.ptr(w), k, n, Q6_K, m)
-        return _held(rocm)
+        return scratch_held(rocm)
 
-    assert 4 * m * k <= _fresh_thread(body) <= 512 << 20
+    assert 4 * m * k <= fresh_thread(body) <= 512 << 20
     assert not y.any()
 
 
@@ -282,9 +255,9 @@ def test_prompt_panels(rocm, dev, oracle, t, ns, k, m):
     def body():
         rocm.call("aljabr_rocm_matvec_tb_triple_batch", *[dev.ptr(y) for y in ys], dev.ptr(xd),
                   *[dev.ptr(w) for w in ws], k, *ns, t, t, t, m)
-        return _held(rocm)
+        return scratch_held(rocm)
 
-    assert _fresh_thread(body) >= (64 << 20) + 4 * m * k
+    assert fresh_thread(body) >= (64 << 20) + 4 * m * k
     g = np.random.default_rng(1)
     for y, raw, n in zip(ys, raws, ns):
         got = dev.get(y).reshape(m, n)
