@@ -5,6 +5,18 @@
 #include "prompt_gemm.hpp"
 
 namespace aljabr {
+
+template <> void prompt_pack<kPgNF4>(const PgArgs &, hipStream_t);
+template <> void prompt_pack<kPgQ40>(const PgArgs &, hipStream_t);
+template <> void prompt_pack<kPgQ80>(const PgArgs &, hipStream_t);
+template <> void prompt_pack<kPgQ4K>(const PgArgs &, hipStream_t);
+template <> void prompt_pack<kPgQ6K>(const PgArgs &, hipStream_t);
+template <> void prompt_multiply<kPgNF4>(const PgArgs &, int, int, hipStream_t);
+template <> void prompt_multiply<kPgQ40>(const PgArgs &, int, int, hipStream_t);
+template <> void prompt_multiply<kPgQ80>(const PgArgs &, int, int, hipStream_t);
+template <> void prompt_multiply<kPgQ4K>(const PgArgs &, int, int, hipStream_t);
+template <> void prompt_multiply<kPgQ6K>(const PgArgs &, int, int, hipStream_t);
+
 namespace {
 
 using pg::half8;
@@ -92,35 +104,6 @@ __global__ __launch_bounds__(256) void prompt_sum_kernel(PgArgs a) {
     (s == 0 ? a.y[0] : s == 1 ? a.y[1] : a.y[2])[static_cast<size_t>(m) * rows + (n - start)] = static_cast<float>(v);
 }
 
-// The power of two that brings a token row's largest finite magnitude into
-// [2^8, 2^9): with it any fp32 row fits the fp16 parts. One workgroup a row.
-__global__ __launch_bounds__(256) void prompt_scale_kernel(const float *x, float *scale, int K) {
-    __shared__ float best[4];
-    const float4 *row = reinterpret_cast<const float4 *>(x + static_cast<size_t>(blockIdx.x) * K);
-    const int quads = K >> 2;                            // K % 32 == 0
-    float top = 0.0f;
-    for (int k0 = threadIdx.x; k0 < quads; k0 += 4 * 256) {
-        float4 v[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = k0 + 256 * i < quads ? row[k0 + 256 * i] : float4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float e[4] = {fabsf(v[i].x), fabsf(v[i].y), fabsf(v[i].z), fabsf(v[i].w)};
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                if (e[j] <= 3.4028235e38f) top = fmaxf(top, e[j]);
-        }
-    }
-    top = wave_max(top);
-    if ((threadIdx.x & 63) == 0) best[threadIdx.x >> 6] = top;
-    __syncthreads();
-    if (threadIdx.x) return;
-    top = fmaxf(fmaxf(best[0], best[1]), fmaxf(best[2], best[3]));
-    int e = 9;
-    if (top > 0.0f) (void)frexpf(top, &e);           // top in [2^(e-1), 2^e)
-    scale[blockIdx.x] = ldexpf(1.0f, (e < -100 ? -100 : e) - 9);
-}
-
 // What a call holds of the stream's scratch: the activation image of a pass of
 // tokens, the weight image of a panel of rows, the K slices' partial sums over
 // all panels.
@@ -176,6 +159,26 @@ Plan make_plan(int f, int xp, int M, int N, int all, int chunks, int cus) {
         }
     }
     return best;
+}
+
+void pack_panel(int f, const PgArgs &a, hipStream_t s) {
+    switch (f) {
+    case kPgNF4: return prompt_pack<kPgNF4>(a, s);
+    case kPgQ40: return prompt_pack<kPgQ40>(a, s);
+    case kPgQ80: return prompt_pack<kPgQ80>(a, s);
+    case kPgQ4K: return prompt_pack<kPgQ4K>(a, s);
+    default: return prompt_pack<kPgQ6K>(a, s);
+    }
+}
+
+void multiply_panel(int f, const PgArgs &a, int xp, int mt, hipStream_t s) {
+    switch (f) {
+    case kPgNF4: return prompt_multiply<kPgNF4>(a, xp, mt, s);
+    case kPgQ40: return prompt_multiply<kPgQ40>(a, xp, mt, s);
+    case kPgQ80: return prompt_multiply<kPgQ80>(a, xp, mt, s);
+    case kPgQ4K: return prompt_multiply<kPgQ4K>(a, xp, mt, s);
+    default: return prompt_multiply<kPgQ6K>(a, xp, mt, s);
+    }
 }
 
 // Whether the passes that the call replaces run any of its tokens in fp32:
@@ -246,7 +249,7 @@ int enqueue_prompt_gemm(const RowsOut *outs, int nseg, const float *A, int K, in
     const auto layout = [&](const Plan &p, int mm) {
         const size_t tiles = static_cast<size_t>(p.mt_groups) * p.mt;
         return Layout{a.chunks * tiles * 4096, f == kPgQ4K ? (a.chunks / 4) * tiles * 1024 : 0,
-                      scaled ? (static_cast<size_t>(mm) * sizeof(float) + 255) & ~size_t{255} : 0,
+                      scaled ? tiles * 32 * sizeof(float) : 0,
                       p.slices > 1 ? static_cast<size_t>(p.slices) * mm * a.N * sizeof(float) : 0};
     };
     const auto plan = [&](int mm) { return make_plan(f, xparts, mm, std::min(panel * 32, a.N), a.N, a.chunks, cus); };
@@ -275,30 +278,23 @@ int enqueue_prompt_gemm(const RowsOut *outs, int nseg, const float *A, int K, in
         a.xl = xl;
         a.sums = sums ? next : nullptr;
         a.codes = next + sums;
-        float *scale = scaled ? reinterpret_cast<float *>(next + sums + image) : nullptr;
-        a.scale = scale;
+        a.scale = scaled ? reinterpret_cast<const float *>(next + sums + image) : nullptr;
         a.part = parts ? reinterpret_cast<float *>(next + sums + image + scales) : nullptr;
         for (int i = 0; i < nseg; ++i) a.y[i] = outs[i].y + static_cast<size_t>(m0) * outs[i].n;
         const float *x = A + static_cast<size_t>(m0) * K;
-        if (scaled) hipLaunchKernelGGL(prompt_scale_kernel, dim3(mm), dim3(256), 0, s, x, scale, K);
-        hipLaunchKernelGGL(prompt_pack_kernel, dim3(static_cast<unsigned>(a.chunks * a.tiles)), dim3(256), 0, s,
-                           x, reinterpret_cast<u32x4 *>(buf),
-                           reinterpret_cast<u32x4 *>(xl),
-                           reinterpret_cast<_Float16 *>(const_cast<uint8_t *>(a.sums)), mm, K, a.tiles, f == kPgNF4,
-                           static_cast<const float *>(scale));
+        a.x = x;
         for (a.tile0 = 0; a.tile0 < all_tiles; a.tile0 += panel) {
             a.ntiles = std::min(panel, all_tiles - a.tile0);
             a.n_groups = (a.ntiles + 2 * kPgWaves - 1) / (2 * kPgWaves);
             a.aux = reinterpret_cast<const uint32_t *>(a.codes + a.ntiles * tile_codes);
-            int rc = ALJABR_ROCM_OK;
-            switch (f) {
-            case kPgNF4: rc = prompt_launch_nf4(a, xparts, p.mt, s); break;
-            case kPgQ40: rc = prompt_launch_q40(a, p.mt, s); break;
-            case kPgQ80: rc = prompt_launch_q80(a, p.mt, s); break;
-            case kPgQ4K: rc = prompt_launch_q4k(a, xparts, p.mt, s); break;
-            default: rc = prompt_launch_q6k(a, p.mt, s); break;
-            }
-            if (rc != ALJABR_ROCM_OK) return rc;
+            a.scale_rows = scaled && a.tile0 == 0 ? mm : 0;
+            pack_panel(f, a, s);
+            if (a.tile0 == 0)
+                hipLaunchKernelGGL(prompt_pack_kernel, dim3(static_cast<unsigned>(a.chunks * a.tiles)), dim3(256), 0, s, x,
+                                   reinterpret_cast<u32x4 *>(buf), reinterpret_cast<u32x4 *>(xl),
+                                   reinterpret_cast<_Float16 *>(const_cast<uint8_t *>(a.sums)), mm, K, a.tiles,
+                                   f == kPgNF4, a.scale);
+            multiply_panel(f, a, xparts, p.mt, s);
         }
         if (a.part)
             hipLaunchKernelGGL(prompt_sum_kernel, dim3(static_cast<unsigned>((a.N + 255) / 256), static_cast<unsigned>(mm)),

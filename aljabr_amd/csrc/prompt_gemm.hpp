@@ -65,13 +65,14 @@ struct PgArgs {
     int tile0, ntiles;                           // row tiles of this panel
     const uint8_t *xh, *xl;                      // activation image [chunk][token tile][step][lane] x 16 bytes
     const uint8_t *sums;                         // Q4_K: [super-block][token tile][lane] x 16 bytes
-    const float *scale;                          // [M] powers of two the image's rows were divided by, or null
+    const float *scale;                          // [tokens of the image] powers of two its rows were divided by, or null
+    const float *x;                              // [M][K], for the row scales
+    int scale_rows;                              // rows whose scale the weight image's launch writes
     float *part;                                 // [slice][M][N] with several K slices, else null
     int M, N, K;
     int chunks;                                  // ceil(K / 64)
     int per;                                     // chunks per K slice (a multiple of 4 for the K-quants)
     int slices, tiles, mt_groups, n_groups;      // token tiles of the image, workgroup grid
-    int add;
 };
 
 namespace pg {
@@ -316,15 +317,51 @@ __device__ __forceinline__ void dma4_at(const void *base, uint32_t offset, uint3
                  : "memory");
 }
 
+// The power of two that brings a token row's largest finite magnitude into
+// [2^8, 2^9): with it any fp32 row fits the fp16 parts.
+__device__ __forceinline__ void row_scale(const float *x, int K, float *scale) {
+    __shared__ float best[4];
+    const float4 *row = reinterpret_cast<const float4 *>(x);
+    const int quads = K >> 2;                            // K % 32 == 0
+    float top = 0.0f;
+    for (int k0 = threadIdx.x; k0 < quads; k0 += 4 * 256) {
+        float4 v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = k0 + 256 * i < quads ? row[k0 + 256 * i] : float4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float e[4] = {fabsf(v[i].x), fabsf(v[i].y), fabsf(v[i].z), fabsf(v[i].w)};
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (e[j] <= 3.4028235e38f) top = fmaxf(top, e[j]);
+        }
+    }
+    top = wave_max(top);
+    if ((threadIdx.x & 63) == 0) best[threadIdx.x >> 6] = top;
+    __syncthreads();
+    if (threadIdx.x) return;
+    top = fmaxf(fmaxf(best[0], best[1]), fmaxf(best[2], best[3]));
+    int e = 9;
+    if (top > 0.0f) (void)frexpf(top, &e);               // top in [2^(e-1), 2^e)
+    *scale = ldexpf(1.0f, (e < -100 ? -100 : e) - 9);
+}
+
 // Weights -> image: one workgroup per row tile and four chunks, a wave each
-// (the lines of a row are read by one workgroup at a time).
+// (the lines of a row are read by one workgroup at a time). The first
+// `scale_rows` workgroups write a token row's scale each: it is needed after
+// this launch, and a launch of its own took 4 to 8 us more.
 template <int F>
-__global__ __launch_bounds__(256) void prompt_weights_kernel(PgArgs a, uint8_t *codes, uint32_t *aux) {
+__global__ __launch_bounds__(256) void prompt_weights_kernel(PgArgs a, uint8_t *codes, uint32_t *aux, float *scale) {
     using R = Raw<F>;
+    if (static_cast<int>(blockIdx.x) < a.scale_rows) {
+        row_scale(a.x + static_cast<size_t>(blockIdx.x) * a.K, a.K, scale + blockIdx.x);
+        return;
+    }
+    const int item = blockIdx.x - a.scale_rows;
     const int lane = threadIdx.x & 63, h = lane >> 5, i = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int quads = (a.chunks + 3) >> 2;
-    const int tile = blockIdx.x / quads, quad = blockIdx.x % quads;
+    const int tile = item / quads, quad = item % quads;
     const int kb = 4 * quad + wave;
     if (kb >= a.chunks) return;
     const int r = (a.tile0 + tile) * 32;
@@ -414,8 +451,8 @@ __device__ __forceinline__ void pace() {
 }
 
 // One wave per SIMD where the LDS takes one workgroup a CU (four token tiles;
-// two for NF4, Q6_K): the wave overlaps its own work in 256 VGPRs, and its
-// earlier sums (tot) stay in AGPRs. Its tiles run one after the other, each tile's products (US steps into one
+// two for NF4, Q6_K): the wave overlaps its own work in 256 VGPRs, and what
+// does not fit or rests (tot) is in AGPRs. Its tiles run one after the other, each tile's products (US steps into one
 // fresh accumulator tile) issued while the vector ALU scales the previous
 // tile's products into acc and decodes fragments of the next US steps;
 // weights and activations arrive two chunks ahead by LDS-DMA, every wait for
@@ -549,14 +586,15 @@ __global__ __launch_bounds__(kPgThreads, (PgLds<F, XP, MT, NT>::kSimdWaves)) voi
 #pragma unroll
     for (int j = 0; j < US; ++j) read_x(x[0][j], 0, 0, 0, j);
 
-    // The sums of earlier chunks. acc itself runs over kFold chunks only (half
-    // of that in short slices): one fp32 chain over all of K rounds more than
-    // the waves and slices of the passes do. Error against float64 of the
-    // passes, one chain, this: Q8_0 4096 x 14336, 512 tokens 1.18e-7, 2.08e-7,
-    // 1.10e-7; K = 1024 0.98, 1.25, 0.94; NF4 (of fp16(x)) K = 14336 1.42,
-    // 2.12, 1.19. It costs 2 to 5 % of the time at four token tiles.
-    constexpr int kFold = 8;
-    const int step = kb1 - kb0 <= 2 * kFold ? kFold / 2 : kFold;
+    // Two parts: the sums of earlier chunks. acc itself runs over kFold chunks
+    // only (half of that in short slices): one fp32 chain over all of K rounds
+    // more than the waves and slices of the passes do. Error against float64 of
+    // the passes, one chain, this: Q8_0 4096 x 14336, 512 tokens 1.18e-7,
+    // 2.08e-7, 1.10e-7; K = 1024 0.98, 1.25, 0.94. The passes of NF4 and Q6_K
+    // round more (1.9e-7 to 2.1e-7): half as many folds. They cost 2 to 8 % of
+    // the time at four token tiles. One part is rounded to 2e-4 anyway: none.
+    constexpr int kFold = F == kPgNF4 || F == kPgQ6K ? 16 : 8;
+    const int step = XP == 1 ? a.chunks : kb1 - kb0 <= 2 * kFold ? kFold / 2 : kFold;
     f32x16 tot[MT][NT];
 #pragma unroll
     for (int m = 0; m < MT; ++m)
@@ -647,6 +685,7 @@ __global__ __launch_bounds__(kPgThreads, (PgLds<F, XP, MT, NT>::kSimdWaves)) voi
             chunk(kb, r, r1, r2);
             r = r1;
         }
+        if constexpr (XP == 1) continue;
         // acc goes on with what the addition to tot rounded off.
 #pragma unroll
         for (int m = 0; m < MT; ++m)
@@ -661,29 +700,53 @@ __global__ __launch_bounds__(kPgThreads, (PgLds<F, XP, MT, NT>::kSimdWaves)) voi
                     tot[m][n][q] = sum;
                 }
     }
+    if constexpr (XP == 1) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int n = 0; n < NT; ++n) tot[m][n] = acc[m][n];
+    }
     // The last tile's products; nothing may still be landing in LDS at the end.
 #pragma unroll
     for (int q = 0; q < 16; ++q) tot[MT - 1][NT - 1][q] = fmaf(s_prev, t[1][q], tot[MT - 1][NT - 1][q]);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
     // Column i of each tile: one stacked row.
+    float *dst[NT];
+    size_t ld[NT];
+    bool mine[NT];
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
         const int row = (a.tile0 + rt0 + n) * 32;
-        if (rt0 + n >= a.ntiles || row + i >= a.N) continue;
+        mine[n] = rt0 + n < a.ntiles && row + i < a.N;
         int s = (row >= a.end[0]) + (row >= a.end[1]);
         if (s > a.nseg - 1) s = a.nseg - 1;
         const int start = s == 0 ? 0 : s == 1 ? a.end[0] : a.end[1];
         const int rows = (s == 0 ? a.end[0] : s == 1 ? a.end[1] : a.end[2]) - start;
-        float *dst = a.part ? a.part + static_cast<size_t>(slice) * a.M * a.N + row + i
-                            : (s == 0 ? a.y[0] : s == 1 ? a.y[1] : a.y[2]) + (row - start + i);
-        const size_t ld = a.part ? a.N : rows;
+        dst[n] = a.part ? a.part + static_cast<size_t>(slice) * a.M * a.N + row + i
+                        : (s == 0 ? a.y[0] : s == 1 ? a.y[1] : a.y[2]) + (row - start + i);
+        ld[n] = a.part ? a.N : rows;
+    }
 #pragma unroll
-        for (int m = 0; m < MT; ++m) {
+    for (int m = 0; m < MT; ++m) {
+        const int tok0 = (mg * MT + m) * 32 + 4 * h;
+        if (a.scale) {                           // four of a tile's tokens at a time, not a load before every store
+            float4 f[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) f[q] = *reinterpret_cast<const float4 *>(a.scale + tok0 + 8 * q);
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+#pragma unroll
+                for (int q = 0; q < 16; ++q)
+                    tot[m][n][q] *= (q & 3) == 0 ? f[q >> 2].x : (q & 3) == 1 ? f[q >> 2].y : (q & 3) == 2 ? f[q >> 2].z : f[q >> 2].w;
+        }
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+            if (!mine[n]) continue;
 #pragma unroll
             for (int q = 0; q < 16; ++q) {
-                const int tok = (mg * MT + m) * 32 + 8 * (q >> 2) + 4 * h + (q & 3);
-                if (tok < a.M) dst[static_cast<size_t>(tok) * ld] = a.scale ? tot[m][n][q] * a.scale[tok] : tot[m][n][q];
+                const int tok = tok0 + 8 * (q >> 2) + (q & 3);
+                if (tok < a.M) dst[n][static_cast<size_t>(tok) * ld[n]] = tot[m][n][q];
             }
         }
     }
@@ -692,13 +755,13 @@ __global__ __launch_bounds__(kPgThreads, (PgLds<F, XP, MT, NT>::kSimdWaves)) voi
 template <int F>
 void pack_weights(const PgArgs &a, hipStream_t s) {
     const int quads = (a.chunks + 3) / 4;
-    hipLaunchKernelGGL((prompt_weights_kernel<F>), dim3(static_cast<unsigned>(a.ntiles * quads)), dim3(256), 0, s, a,
-                       const_cast<uint8_t *>(a.codes), const_cast<uint32_t *>(a.aux));
+    hipLaunchKernelGGL((prompt_weights_kernel<F>), dim3(static_cast<unsigned>(a.ntiles * quads + a.scale_rows)), dim3(256), 0,
+                       s, a, const_cast<uint8_t *>(a.codes), const_cast<uint32_t *>(a.aux), const_cast<float *>(a.scale));
 }
 
 // Launch of one instantiation (the LDS attribute is per kernel, per process).
 template <int F, int XP, int MT, int NT, int US>
-int launch(const PgArgs &a, hipStream_t s) {
+void launch(const PgArgs &a, hipStream_t s) {
     const auto fn = prompt_gemm_kernel<F, XP, MT, NT, US>;
     constexpr uint32_t lds = PgLds<F, XP, MT, NT>::kBytes;
     static std::atomic<bool> set{false};
@@ -708,19 +771,14 @@ int launch(const PgArgs &a, hipStream_t s) {
         set.store(true, std::memory_order_release);
     }
     const int total = a.n_groups * a.slices * a.mt_groups;
-    pack_weights<F>(a, s);
     hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(8 * ((total + 7) / 8))), dim3(kPgThreads), lds, s, a);
-    return ALJABR_ROCM_OK;
 }
 
 }  // namespace pg
 
-// One launch per format file: mt (2 or 4) x 2 tiles per wave, xp activation
-// parts.
-int prompt_launch_nf4(const PgArgs &a, int xp, int mt, hipStream_t s);
-int prompt_launch_q40(const PgArgs &a, int mt, hipStream_t s);
-int prompt_launch_q80(const PgArgs &a, int mt, hipStream_t s);
-int prompt_launch_q4k(const PgArgs &a, int xp, int mt, hipStream_t s);
-int prompt_launch_q6k(const PgArgs &a, int mt, hipStream_t s);
+// Per format file: the weight image of a panel, and the GEMM with mt (2 or 4)
+// x 2 tiles per wave and xp activation parts.
+template <int F> void prompt_pack(const PgArgs &a, hipStream_t s);
+template <int F> void prompt_multiply(const PgArgs &a, int xp, int mt, hipStream_t s);
 
 }  // namespace aljabr

@@ -3,8 +3,10 @@
 
 namespace aljabr {
 
-int prompt_launch_q80(const PgArgs &a, int mt, hipStream_t s) {
-    return mt == 4 ? pg::launch<kPgQ80, 2, 4, 2, 2>(a, s) : pg::launch<kPgQ80, 2, 2, 2, 2>(a, s);
+template <> void prompt_pack<kPgQ80>(const PgArgs &a, hipStream_t s) { pg::pack_weights<kPgQ80>(a, s); }
+
+template <> void prompt_multiply<kPgQ80>(const PgArgs &a, int , int mt, hipStream_t s) {
+    mt == 4 ? pg::launch<kPgQ80, 2, 4, 2, 2>(a, s) : pg::launch<kPgQ80, 2, 2, 2, 2>(a, s);
 }
 
 }  // namespace aljabr
