@@ -62,17 +62,23 @@ int enqueue_matmul_multi(float *const *C, const float *A, const uint8_t *const *
         if (enqueue_rows_fused(type[0], outs, n, A, nullptr, 0.0f, K, 0, kRowsStore) == ALJABR_ROCM_OK)
             return ALJABR_ROCM_OK;
     }
-    if (same && prompt_gguf(type[0], batch, N[0], K)) {
+    if (same && batch >= 2) {
         RowsOut outs[3];
         const int xparts = prompt_xparts(type[0], N[0], K);
-        // One precision for the stack, and no last token beside it.
-        bool stack = prompt_last_token(xparts, batch) == 0;
+        const int last = prompt_last_token(xparts, batch);
+        bool stack = true;                       // one precision for the stack
         for (int i = 0; i < n; ++i) {
             outs[i] = RowsOut{C[i], B[i], nullptr, N[i]};
-            stack = stack && prompt_gguf(type[0], batch, N[i], K) && prompt_xparts(type[0], N[i], K) == xparts;
+            stack = stack && prompt_xparts(type[0], N[i], K) == xparts;
         }
-        if (stack) {
-            const int rc = enqueue_prompt_gemm(outs, n, A, K, type[0], xparts, batch);
+        if (stack && prompt_gguf(type[0], batch - last, N, n, K, xparts)) {
+            const int rc = enqueue_prompt_gemm(outs, n, A, K, type[0], xparts, batch - last);
+            if (rc == ALJABR_ROCM_OK && last) {
+                const size_t m0 = static_cast<size_t>(batch - 1);
+                float *c[3];
+                for (int i = 0; i < n; ++i) c[i] = C[i] + m0 * N[i];
+                return enqueue_matmul_multi(c, A + m0 * K, B, K, N, type, n, 1);
+            }
             if (rc != ALJABR_ROCM_ERR_UNSUPPORTED) return rc;
         }
     }

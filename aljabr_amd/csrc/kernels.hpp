@@ -235,9 +235,9 @@ int enqueue_prompt_gemm(const RowsOut *outs, int nseg, const float *A, int K, in
 // Whether the passes of up to 32 tokens round the activations of a Q4_K
 // matrix to fp16 (q4k_gemm_pass takes its shape).
 bool q4k_rounds_activations(int N, int K);
-// Whether M tokens of a GGUF type are a prompt, and the activation parts its
-// GEMM takes (those of the passes it replaces).
-bool prompt_gguf(int type, int M, int N, int K);
+// Whether the prompt GEMM takes M tokens of n stacked matrices of a GGUF type,
+// and its activation parts (those of the passes it replaces).
+bool prompt_gguf(int type, int M, const int *N, int n, int K, int xparts);
 int prompt_xparts(int type, int N, int K);
 // Tokens of a GGUF prompt with rounded activations that run on the batch-1
 // kernel instead: the single one that the passes of 32 leave over, in fp32.

@@ -458,28 +458,92 @@ using namespace aljabr;
 
 namespace aljabr {
 
-// Where the prompt GEMM (a pass over the weights to lay them out, then one
-// for all tokens) beats the passes of 8, 32 or 64 tokens, in us per FFN of
-// three matrices, passes against prompt GEMM:
-//   Q4_0/Q8_0 1024 x 2816    12 tokens 56/34;  2560 x 7680 12: 90/68;
-//             4096 x 14336   16: 112/132, 24: 168/133
-//   Q4_K/Q6_K 1024 x 2816    33: 93/42;  2560 x 7680 (Q6_K) 33: 99/93;
-//             4096 x 14336   48: 145/144, 65: 193/182;
-//             Q/K/V of 1024  33: 35/48, 128: 105/50 (three small launches)
-//   NF4       1024 x 2816    128: 64/64, 192: 95/70;  2048 x 5632 129: 127/97;
-//             4096 x 14336   129: 222/228, 192: 268/243
-//             2560 x 7680    65: 129/102 (the passes split the activations)
-static constexpr long long kLargeMatrix = 32LL << 20, kSmallMatrix = 2LL << 20;   // N * K
+// Where the prompt GEMM (a pass over the weights to lay them out, then one for
+// all tokens) beats the passes it replaces. Both are priced in us from sweeps
+// over N x K from 64 x 1024 to 128256 x 4096 and 9 to 129 tokens; at M tokens
+// of one matrix (or Q/K/V), passes against prompt GEMM:
+//   Q4_0  1024 x 1024  16: 15/14, 17: 19/15     4096 x 4096   17: 22/26, 18: 25/25
+//         14336 x 4096 17: 43/46, 18: 50/46     Q/K/V of 4096 17: 63/30
+//   Q8_0  2560 x 2560  16: 19/22, 17: 24/23     128256 x 4096 25: 495/504, 33: 624/508
+//         3328 x 1280   9: 27/18 (fp32)         Q/K/V of 2560  9: 38/23
+//   Q4_K  1024 x 1024  64: 17/18, 65: 19/18     4096 x 4096   66: 30/32, 97: 37/33
+//         1280 x 1280   9: 10/17, 17: 18/17 (fp32)
+//   Q6_K  5632 x 2048  65: 32/33, 66: 35/32     14336 x 4096  65: 88/97, 66: 98/96
+//         3328 x 1280   9: 19/22, 16: 29/22 (fp32)
+namespace {
 
-bool prompt_gguf(int type, int M, int N, int K) {
-    const long long size = static_cast<long long>(N) * K;
-    if (type == ALJABR_ROCM_TYPE_Q4_K || type == ALJABR_ROCM_TYPE_Q6_K)
-        return M > (size >= kLargeMatrix || size < kSmallMatrix ? 64 : 32);
-    return (type == ALJABR_ROCM_TYPE_Q4_0 || type == ALJABR_ROCM_TYPE_Q8_0) && M > (size >= kLargeMatrix ? 16 : 8);
+float mega(int N, int K) { return static_cast<float>(N) * static_cast<float>(K) / (1 << 20); }
+
+bool k_quant(int type) { return type == ALJABR_ROCM_TYPE_Q4_K || type == ALJABR_ROCM_TYPE_Q6_K; }
+
+// One pass over an N x K matrix: 8 tokens in fp32 (K % 512 != 0), else on the
+// matrix cores 8 (Q4_0, Q8_0) or 32 (K-quants; their LDS-staged kernel's time
+// goes with the row tiles that its workgroups run in turn, kq_launch).
+float pass_us(int type, int N, int K, int xparts) {
+    const float mi = mega(N, K);
+    if (K % 512 != 0)
+        return type == ALJABR_ROCM_TYPE_Q4_K   ? 4.5f + 2.05f * mi
+               : type == ALJABR_ROCM_TYPE_Q6_K ? 6.0f + 2.3f * mi
+                                               : 6.7f + 3.7f * mi;
+    if (type == ALJABR_ROCM_TYPE_Q4_K && xparts == 1) return 8.0f + 0.235f * mi;
+    const bool q4 = type == ALJABR_ROCM_TYPE_Q4_K;
+    const long long cus = device_cu_count() > 0 ? device_cu_count() : 256;
+    const long long units = (N + 127LL) / 128 * (K / 512);
+    const bool one = units <= cus;               // one row tile a workgroup
+    if (type == ALJABR_ROCM_TYPE_Q4_0) return one ? 7.5f + 0.07f * mi : 8.0f + 0.18f * mi;
+    if (type == ALJABR_ROCM_TYPE_Q8_0) return one ? 8.2f + 0.12f * mi : 10.5f + 0.19f * mi;
+    if (one) return q4 ? 8.0f + 0.2f * mi : 10.0f + 0.15f * mi;
+    const long long nt = (units + 1) / 2 <= cus || !q4 ? 2 : 4;
+    const float tiles = static_cast<float>(((units + nt - 1) / nt + cus - 1) / cus * nt);
+    return q4 ? 1.5f + 7.0f * tiles : 5.0f + 7.7f * tiles;
 }
 
+// Passes for M tokens; a last single token takes the batch-1 kernel.
+float pass_count(int type, int M, int K) {
+    const int per = K % 512 == 0 && k_quant(type) ? 32 : 8, rest = M % per;
+    const float last = rest == 0        ? 0.0f
+                       : K % 512 != 0 ? 0.1f + 0.125f * static_cast<float>(rest)
+                       : rest > 1     ? 1.0f
+                                      : (type == ALJABR_ROCM_TYPE_Q8_0 ? 0.65f : 0.5f);
+    return static_cast<float>(M / per) + last;
+}
+
+// Up to 64 or about 130 tokens; past 80 Mi the images leave the cache. The
+// margin of what the two fits miss is part of it.
+float prompt_us(int type, int M, float mi, int xparts) {
+    const float far = mi > 80.0f ? mi - 80.0f : 0.0f;
+    const bool few = M <= 64;                    // half the token tiles
+    switch (type) {
+    case ALJABR_ROCM_TYPE_Q4_0: return 1.05f * (14.5f + 0.55f * mi);
+    case ALJABR_ROCM_TYPE_Q8_0: return 1.05f * (14.0f + 0.78f * mi + 0.25f * far);
+    case ALJABR_ROCM_TYPE_Q4_K: return 1.1f * (17.0f + (few ? 0.65f : xparts == 1 ? 0.7f : 0.85f) * mi + 0.1f * far);
+    default: return 18.0f + (few ? 1.15f : 1.4f) * mi + 0.12f * far;
+    }
+}
+
+}  // namespace
+
+bool prompt_gguf(int type, int M, const int *N, int n, int K, int xparts) {
+    if (!k_quant(type) && type != ALJABR_ROCM_TYPE_Q4_0 && type != ALJABR_ROCM_TYPE_Q8_0) return false;
+    // One pass takes them all, in one launch for a stack.
+    if (M <= (K % 512 == 0 && k_quant(type) ? 32 : 8)) return false;
+    float passes = 0.0f, mi = 0.0f;
+    for (int i = 0; i < n; ++i) {
+        passes += pass_us(type, N[i], K, xparts);
+        mi += mega(N[i], K);
+    }
+    return pass_count(type, M, K) * passes > prompt_us(type, M, mi, xparts);
+}
+
+// NF4: passes of 64. At K of 1024 and multiples of 4096 and N > 2 K (gate, up)
+// two passes and a third of up to 64 tokens beat the prompt GEMM's grid.
+//   1024 x 1024  128: 13/16, 129: 19/16        2816 x 1024   192: 20/22, 256: 27/24
+//   4096 x 4096  128: 30/30, 129: 38/34        14336 x 4096  160: 76/81, 256: 116/91
+//   8192 x 3072  129: 55/46                    4096 x 14336  128: 61/61, 129: 78/74
+// K % 1024 != 0: the passes split the activations or run in fp32.
+//   640 x 2560    65: 25/19                    9984 x 3328    65: 56/46
 static bool prompt_nf4(int M, int N, int K) {
-    return M > (K % 1024 != 0 ? 64 : static_cast<long long>(N) * K >= kLargeMatrix ? 144 : 128);
+    return M > (K % 1024 != 0 ? 64 : N > 2LL * K && (K == 1024 || K % 4096 == 0) ? 192 : 128);
 }
 
 // M > 8 slices run the small-M kernels per slice of 8 tokens (weights are
@@ -527,7 +591,7 @@ int enqueue_matmul_gguf(float *C, const float *A, const uint8_t *B, int K, int N
                         size_t part_floats) {
     const int xparts = prompt_xparts(type, N, K);
     const int last = prompt_last_token(xparts, M);
-    if (!part && prompt_gguf(type, M - last, N, K)) {
+    if (!part && prompt_gguf(type, M - last, &N, 1, K, xparts)) {
         const RowsOut o{C, B, nullptr, N};
         const int rc = enqueue_prompt_gemm(&o, 1, A, K, type, xparts, M - last);
         if (rc == ALJABR_ROCM_OK && last) {

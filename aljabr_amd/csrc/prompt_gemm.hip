@@ -89,19 +89,20 @@ __device__ __forceinline__ double slice_sum_f64(const float *p, size_t stride, i
     return acc;
 }
 
-__global__ __launch_bounds__(256) void prompt_sum_kernel(PgArgs a) {
+// The arguments fill the 14 preloaded dwords.
+__global__ __launch_bounds__(256) void prompt_sum_kernel(const float *part, int M, int N, int slices, int nseg, float *y0,
+                                                         float *y1, float *y2, int end0, int end1) {
     const int n = blockIdx.x * 256 + threadIdx.x, m = blockIdx.y;
-    if (n >= a.N) return;
-    const float *p = a.part + static_cast<size_t>(m) * a.N + n;
-    const size_t stride = static_cast<size_t>(a.M) * a.N;
-    const double v = a.slices <= 4   ? slice_sum_f64<4>(p, stride, a.slices)
-                     : a.slices <= 8 ? slice_sum_f64<8>(p, stride, a.slices)
-                                     : slice_sum_f64<16>(p, stride, a.slices);
-    int s = (n >= a.end[0]) + (n >= a.end[1]);
-    if (s > a.nseg - 1) s = a.nseg - 1;
-    const int start = s == 0 ? 0 : s == 1 ? a.end[0] : a.end[1];
-    const int rows = (s == 0 ? a.end[0] : s == 1 ? a.end[1] : a.end[2]) - start;
-    (s == 0 ? a.y[0] : s == 1 ? a.y[1] : a.y[2])[static_cast<size_t>(m) * rows + (n - start)] = static_cast<float>(v);
+    if (n >= N) return;
+    const float *p = part + static_cast<size_t>(m) * N + n;
+    const size_t stride = static_cast<size_t>(M) * N;
+    const double v = slices <= 4   ? slice_sum_f64<4>(p, stride, slices)
+                     : slices <= 8 ? slice_sum_f64<8>(p, stride, slices)
+                                   : slice_sum_f64<16>(p, stride, slices);
+    const int s = min((n >= end0) + (n >= end1), nseg - 1);
+    const int start = s == 0 ? 0 : s == 1 ? end0 : end1;
+    const int rows = (s == nseg - 1 ? N : s == 0 ? end0 : end1) - start;
+    (s == 0 ? y0 : s == 1 ? y1 : y2)[static_cast<size_t>(m) * rows + (n - start)] = static_cast<float>(v);
 }
 
 // What a call holds of the stream's scratch: the activation image of a pass of
@@ -298,7 +299,7 @@ int enqueue_prompt_gemm(const RowsOut *outs, int nseg, const float *A, int K, in
         }
         if (a.part)
             hipLaunchKernelGGL(prompt_sum_kernel, dim3(static_cast<unsigned>((a.N + 255) / 256), static_cast<unsigned>(mm)),
-                               dim3(256), 0, s, a);
+                               dim3(256), 0, s, a.part, mm, a.N, p.slices, nseg, a.y[0], a.y[1], a.y[2], a.end[0], a.end[1]);
     }
     return ALJABR_ROCM_OK;
 }

@@ -324,12 +324,12 @@ __device__ __forceinline__ void row_scale(const float *x, int K, float *scale) {
     const float4 *row = reinterpret_cast<const float4 *>(x);
     const int quads = K >> 2;                            // K % 32 == 0
     float top = 0.0f;
-    for (int k0 = threadIdx.x; k0 < quads; k0 += 4 * 256) {
-        float4 v[4];
+    for (int k0 = threadIdx.x; k0 < quads; k0 += 8 * 256) {
+        float4 v[8];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = k0 + 256 * i < quads ? row[k0 + 256 * i] : float4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int i = 0; i < 8; ++i) v[i] = row[min(k0 + 256 * i, quads - 1)];   // past the end: the last again
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < 8; ++i) {
             const float e[4] = {fabsf(v[i].x), fabsf(v[i].y), fabsf(v[i].z), fabsf(v[i].w)};
 #pragma unroll
             for (int j = 0; j < 4; ++j)

@@ -15,7 +15,7 @@ import pytest
 from conftest import fresh_thread, rel_l2, scratch_held
 
 pytestmark = pytest.mark.gpu
-Q4_0, Q8_0, Q4_K, Q6_K = 2, 8, 12, 14
+Q4_0, Q8_0, Q4_K, Q6_K, NF4 = 2, 8, 12, 14, 100
 TOL = 2e-6
 
 
@@ -279,3 +279,41 @@ def test_prompt_token_passes(rocm, dev, oracle, m):
     ref = x.astype(np.float64) @ _decoded(oracle, Q8_0, raw, n, k).T
     for i in range(m):
         assert rel_l2(got[i], ref[i]) <= TOL, i
+
+
+# Which path takes a call: the prompt GEMM holds its activation image (2 bytes
+# an element and part) on a stream that had none; the passes' partial sums and
+# images of 8 to 64 tokens are smaller. Both sides of the lines, single
+# matrices and stacks.
+@pytest.mark.parametrize("t,ns,k,m,prompt", [
+    (Q4_0, (4096,), 4096, 17, False), (Q4_0, (4096,), 4096, 25, True), (Q8_0, (4096,), 4096, 9, False),
+    (Q4_0, (4096, 1024, 1024), 4096, 9, True), (Q8_0, (2560, 640, 640), 2560, 17, True), (Q8_0, (1280,), 1280, 9, False),
+    (Q8_0, (3328,), 1280, 9, True), (Q4_K, (4096,), 4096, 64, False), (Q4_K, (4096,), 4096, 98, True),
+    (Q4_K, (1024,), 2048, 33, False), (Q4_K, (1024,), 1024, 66, True), (Q4_K, (4096, 1024, 1024), 4096, 66, True),
+    (Q6_K, (1024,), 1024, 33, False), (Q6_K, (1024,), 1024, 66, True), (Q6_K, (3328,), 1280, 24, True),
+    (NF4, (4096,), 4096, 128, False), (NF4, (4096,), 4096, 160, True), (NF4, (14336,), 4096, 160, False),
+    (NF4, (640,), 2560, 66, True)])
+def test_which_path(rocm, dev, oracle, t, ns, k, m, prompt):
+    import torch
+    x = torch.zeros(m * k, device="cuda:0")
+    ys = [torch.empty(m * n, device="cuda:0") for n in ns]
+    ws = [torch.zeros(n * k * (2 if t == Q8_0 else 1), dtype=torch.uint8, device="cuda:0") for n in ns]
+    absmax = torch.ones(ns[0] * k // 64, device="cuda:0")
+    torch.cuda.synchronize()
+
+    def body():
+        if t == NF4:
+            rocm.call("aljabr_rocm_matvec_tb_batch_nf4", dev.ptr(ys[0]), dev.ptr(x), dev.ptr(ws[0]), dev.ptr(absmax), k,
+                      ns[0], 64, m)
+        elif len(ns) == 1:
+            rocm.call("aljabr_rocm_matvec_tb_batch", dev.ptr(ys[0]), dev.ptr(x), dev.ptr(ws[0]), k, ns[0], t, m)
+        else:
+            rocm.call("aljabr_rocm_matvec_tb_triple_batch", *[dev.ptr(y) for y in ys], dev.ptr(x),
+                      *[dev.ptr(w) for w in ws], k, *ns, t, t, t, m)
+        return scratch_held(rocm)
+
+    held = fresh_thread(body)
+    # Weight image and activation image together.
+    bytes_per = {Q4_0: 0.5625, Q8_0: 1.0625, Q4_K: 0.5625, Q6_K: 1.125, NF4: 0.5625}[t]
+    image = min(sum(ns) * k * bytes_per, 100 << 20) + 2 * m * k
+    assert (held >= image) == prompt, (held, image)
