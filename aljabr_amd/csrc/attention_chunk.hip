@@ -26,7 +26,9 @@
 // Infinities and NaN: zero weights and parts times an infinity would make a
 // NaN that the exact sum does not have, and a masked key's V must not reach a
 // row that cannot see it. A row whose sums are not finite is therefore done
-// again over its own keys in plain fp32.
+// again over its own keys in plain fp32. With an infinite V element that every
+// row sees, 256 rows at 2048 keys take 0.70 ms (the split kernel 0.30 ms
+// whatever the values; 5.3 ms a row and key at a time).
 #include <cmath>
 
 #include "device.hpp"
@@ -45,6 +47,7 @@ constexpr int kThreads = 64 * kWaves;
 constexpr int kRows = 32 * kWaves;           // stacked query rows per workgroup
 constexpr int kKeys = 32;                    // keys per tile
 constexpr int kVtStride = kKeys + 4;         // halves: 72-byte rows, conflict-free 8-byte reads
+constexpr int kRedo = 8;                     // rows that a wave does again together
 constexpr float kLog2eC = 1.4426950408889634f;
 constexpr float kWeightScale = 2048.0f;      // weights are split, and summed over V, times this
 
@@ -289,43 +292,107 @@ __global__ __launch_bounds__(kThreads, 2) void chunk_attention_kernel(ChunkParam
             p.part_ml[(qrow * p.splits + split) * 2 + 1] = l;
         }
     }
-    // Rows that are not finite: the wave does each again, key by key, over the
-    // keys of this split that the row sees.
+    // Rows that are not finite: the wave does them again, kRedo at a time, over
+    // the keys of this split that each sees: a lane per key for the scores (the
+    // rows in LDS, which the tiles have left), a lane per element for the
+    // weights over V.
     uint32_t todo = static_cast<uint32_t>(__ballot(mine && bad));
+    float *qs = reinterpret_cast<float *>(lds) + wave * (kRedo * D);
+    const size_t head = static_cast<size_t>(b * p.Hkv + kvh) * p.Sk * D;
     while (todo) {
-        const int r = __builtin_ctz(todo);
-        todo &= todo - 1;
-        const int rr = w0 + r;
-        const size_t qr = (static_cast<size_t>(b) * p.Hq + kvh * p.G + rr % p.G) * p.Sq + rr / p.G;
-        const int end = min(visible(p, rr / p.G), (kt0 + p.tiles_per_split) * kKeys);
-        const size_t head = static_cast<size_t>(b * p.Hkv + kvh) * p.Sk * D;
-        float mr = -INFINITY, lr = 0.0f, acc[D / 64] = {};
-        for (int key = kt0 * kKeys; key < end; ++key) {
-            float dot = 0.0f;
+        size_t qr[kRedo];
+        int end[kRedo], rows = 0, last = 0;
 #pragma unroll
-            for (int j = 0; j < D / 64; ++j)
-                dot = fmaf(p.q[qr * D + 64 * j + lane] * (p.scale * kLog2eC),
-                           static_cast<float>(p.k[head + static_cast<size_t>(key) * D + 64 * j + lane]), dot);
-            dot = wave_sum(dot);
-            if (dot == -INFINITY) continue;
-            const float mn = fmaxf(mr, dot);
-            const float alpha = mr == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mr - mn);
-            const float w = __builtin_amdgcn_exp2f(dot - mn);
-            lr = fmaf(lr, alpha, w);
-#pragma unroll
-            for (int j = 0; j < D / 64; ++j)
-                acc[j] = fmaf(acc[j], alpha,
-                              w * static_cast<float>(p.v[head + static_cast<size_t>(key) * D + 64 * j + lane]));
-            mr = mn;
+        for (int i = 0; i < kRedo; ++i) {            // past the last row: it again, over no keys
+            const int rr = w0 + (todo ? __builtin_ctz(todo) : 0);
+            qr[i] = (static_cast<size_t>(b) * p.Hq + kvh * p.G + rr % p.G) * p.Sq + rr / p.G;
+            end[i] = todo ? min(visible(p, rr / p.G), (kt0 + p.tiles_per_split) * kKeys) : 0;
+            rows += todo != 0;
+            last = max(last, end[i]);
+            todo &= todo - 1;
         }
-        // A NaN score alone leaves no reference: any finite one carries it.
-        if (mr == -INFINITY && lr != lr) mr = 0.0f;
-        float *dst = p.part_o ? p.part_o + (qr * p.splits + split) * D : p.out + qr * D;
 #pragma unroll
-        for (int j = 0; j < D / 64; ++j) dst[64 * j + lane] = p.part_o ? acc[j] : lr == 0.0f ? 0.0f : acc[j] / lr;
-        if (p.part_o && lane == 0) {
-            p.part_ml[(qr * p.splits + split) * 2] = mr;
-            p.part_ml[(qr * p.splits + split) * 2 + 1] = lr;
+        for (int i = 0; i < kRedo; ++i)
+#pragma unroll
+            for (int j = 0; j < D / 64; ++j) qs[i * D + 64 * j + lane] = p.q[qr[i] * D + 64 * j + lane] * (p.scale * kLog2eC);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // this wave's own writes
+        float mr[kRedo], lr[kRedo], acc[kRedo][D / 64];
+#pragma unroll
+        for (int i = 0; i < kRedo; ++i) {
+            mr[i] = -INFINITY;
+            lr[i] = 0.0f;
+#pragma unroll
+            for (int j = 0; j < D / 64; ++j) acc[i][j] = 0.0f;
+        }
+        for (int k0 = kt0 * kKeys; k0 < last; k0 += 64) {
+            const int key = k0 + lane;
+            const _Float16 *kr = p.k + head + static_cast<size_t>(min(key, p.Sk - 1)) * D;
+            float w[kRedo], dot[kRedo][4] = {};      // four chains: of D / 4 roundings each
+#pragma unroll 1
+            for (int d0 = 0; d0 < D; d0 += 32) {
+                half8 x[4];
+#pragma unroll
+                for (int c = 0; c < 4; ++c) x[c] = *reinterpret_cast<const half8 *>(kr + d0 + 8 * c);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+#pragma unroll
+                    for (int i = 0; i < kRedo; ++i)
+#pragma unroll
+                        for (int e = 0; e < 8; ++e)
+                            dot[i][e & 3] = fmaf(qs[i * D + d0 + 8 * c + e], static_cast<float>(x[c][e]), dot[i][e & 3]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            uint64_t live[kRedo], any = 0, all = ~0ull;   // keys with a weight; the others' V is not touched
+#pragma unroll
+            for (int i = 0; i < kRedo; ++i) {
+                w[i] = (dot[i][0] + dot[i][1]) + (dot[i][2] + dot[i][3]);
+                const bool on = key < end[i] && !(w[i] == -INFINITY);
+                const float mn = fmaxf(mr[i], wave_max(on ? w[i] : -INFINITY));
+                const float alpha = mr[i] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mr[i] - mn);
+                w[i] = on ? __builtin_amdgcn_exp2f(w[i] - mn) : 0.0f;
+                live[i] = __ballot(on);
+                any |= live[i];
+                all &= live[i];
+                lr[i] = fmaf(lr[i], alpha, wave_sum(w[i]));
+#pragma unroll
+                for (int j = 0; j < D / 64; ++j) acc[i][j] *= alpha;
+                mr[i] = mn;
+            }
+#pragma unroll 1
+            for (int c0 = 0; c0 < 64 && any >> c0; c0 += 8) {
+                float v[8][D / 64];
+#pragma unroll
+                for (int c = 0; c < 8; ++c)
+#pragma unroll
+                    for (int j = 0; j < D / 64; ++j)
+                        v[c][j] = static_cast<float>(
+                            p.v[head + static_cast<size_t>(min(k0 + c0 + c, p.Sk - 1)) * D + 64 * j + lane]);
+                const bool whole = (all >> c0 & 0xff) == 0xff;
+#pragma unroll
+                for (int c = 0; c < 8; ++c)
+#pragma unroll
+                    for (int i = 0; i < kRedo; ++i) {
+                        const float wc = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w[i]), c0 + c));
+                        if (whole || (live[i] >> (c0 + c) & 1))
+#pragma unroll
+                            for (int j = 0; j < D / 64; ++j) acc[i][j] = fmaf(wc, v[c][j], acc[i][j]);
+                    }
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < kRedo; ++i) {
+            if (i >= rows) continue;
+            // A NaN score alone leaves no reference: any finite one carries it.
+            if (mr[i] == -INFINITY && lr[i] != lr[i]) mr[i] = 0.0f;
+            float *dst = p.part_o ? p.part_o + (qr[i] * p.splits + split) * D : p.out + qr[i] * D;
+#pragma unroll
+            for (int j = 0; j < D / 64; ++j)
+                dst[64 * j + lane] = p.part_o ? acc[i][j] : lr[i] == 0.0f ? 0.0f : acc[i][j] / lr[i];
+            if (p.part_o && lane == 0) {
+                p.part_ml[(qr[i] * p.splits + split) * 2] = mr[i];
+                p.part_ml[(qr[i] * p.splits + split) * 2 + 1] = lr[i];
+            }
         }
     }
 }
@@ -344,6 +411,10 @@ void launch(const ChunkParams &p, _Float16 *pk, hipStream_t s) {
 //             128 keys, 64: 10.3/14.2
 //   8/8/64    1024 keys, 64: 11.6/14.1;  4096 keys, 32: 19.0/18.2, 64: 34/20
 //   32/4/128  4096 keys: 4: 19.8/20.0, 8: 29/22
+// and at the line (2^27) with several:
+//   32/8/128  8 x 16 rows of Q, 256 keys 26.2/27.1; 4 x 16, 512: 24.5/25.0;
+//             2 x 16, 1024: 24.1/24.4;  64/8/64 (one wave of four with rows)
+//             16 x 4, 512: 26.7/27.4; 16 x 4, 8192: 294/284
 // The line is the split kernel's work (it runs ~7e6 of these products per us,
 // the launches here take ~10 us more), and at least the rows that pay for
 // writing the tile images, a second and third pass over the cache.

@@ -76,6 +76,45 @@ def test_non_finite_rows_stay_apart(rocm, dev, b, sk, where, value):
         assert np.isnan(got[:, :, sq - 10:][up]).all() and np.isfinite(got[:, :, sq - 10:][~up]).all()
 
 
+@pytest.mark.parametrize("hq,hkv,sq,sk,d", [(32, 8, 33, 2050, 128), (8, 8, 129, 1111, 64), (5, 1, 21, 8000, 128)])
+@pytest.mark.parametrize("where", ["q", "v"])
+def test_every_row_done_again(rocm, dev, hq, hkv, sq, sk, d, where):
+    """An infinite V element that all rows of a KV head see, or one NaN row:
+    the other elements, heads and rows keep their accuracy."""
+    q, k, v = _inputs(7, 2, hq, hkv, sq, sk, d)
+    want = _reference(q, k, v, 1)
+    if where == "q":
+        q[1, 1, 2, 5] = np.nan
+    else:
+        v[1, 0, 5, 3] = -np.inf
+    got = _run(rocm, dev, q, k, v, 1)
+    hit = np.zeros(got.shape, bool)
+    if where == "q":
+        hit[1, 1, 2] = True
+        assert np.isnan(got[hit]).all()
+    else:
+        hit[1, :hq // hkv, :, 3] = True
+        assert np.all(got[hit] == -np.inf)
+    assert rel_l2(got[~hit], want[~hit]) <= 1e-6
+
+
+# The chunk kernel's tile image (K, V^T, padded) is on the stream where it took
+# the call; the split kernel's partials are smaller here.
+@pytest.mark.parametrize("b,hq,hkv,sq,sk,d,chunk", [
+    (1, 32, 8, 32, 2048, 128, True), (1, 32, 8, 8, 4097, 128, True), (1, 32, 8, 7, 8192, 128, False),
+    (1, 32, 8, 32, 1000, 128, False), (2, 8, 8, 64, 2048, 128, True), (16, 64, 8, 4, 2048, 64, True)])
+def test_which_kernel(rocm, dev, b, hq, hkv, sq, sk, d, chunk):
+    q, k, v = _inputs(3, b, hq, hkv, sq, sk, d)
+    out, qd, kd, vd = dev.empty(q.size), dev.put(q), dev.put(k), dev.put(v)
+
+    def body():
+        rocm.call("aljabr_rocm_attention_gqa", dev.ptr(out), dev.ptr(qd), dev.ptr(kd), dev.ptr(vd), None, b, hq, hkv, sq,
+                  sk, d, F16, 0.0, 1)
+        return scratch_held(rocm)
+
+    assert (fresh_thread(body) >= 2 * (k.size + v.size)) == chunk
+
+
 def test_growing_calls_rarely_reallocate(rocm, dev):
     """A chunked prompt grows its keys with every call; the stream's scratch
     grows geometrically, not with each (a growth waits for the stream)."""
