@@ -16,16 +16,20 @@
 //      lane-contiguous pieces, two chunks ahead.
 //
 // What bounds it: the matrix cores (32 cycles per product of a 32x32x16
-// step, one to three products per weight), beside which one wave per SIMD
-// issues 16 FMAs per tile and scale group and the decode. NF4 MLP
-// 4096 x 14336: 512 tokens 742 -> 452 us; Q8_0 Q/K/V 3840 x 2560, 197 tokens
-// 727 -> 32 us; Q4_K_M FFN 4096 x 14336, 2048 tokens 5.35 -> 1.45 ms.
+// step, one to three products per weight) and, beside them on one wave per
+// SIMD, the vector ALU (16 FMAs per tile and scale group, the decode). Of a
+// wave's time the matrix cores are busy 59 % (NF4, Q6_K) or 39 % (Q4_K in one
+// part), the vector ALU issues 45 to 50 %; no LDS conflicts. NF4 MLP
+// 4096 x 14336: 512 tokens 742 -> 424 us; Q8_0 Q/K/V 3840 x 2560, 197 tokens
+// 727 -> 31 us; Q4_K_M FFN 4096 x 14336, 2048 tokens 5.35 -> 1.43 ms.
 //
 // Arithmetic, as in the small-M kernels: weights are exact fp16 integers (or
 // NF4's exact H + R level pair, or Q6_K's two exact parts), the block scales
 // stay fp32 on the accumulators, and the activations are one fp16 part (XP =
 // 1, the rounding those kernels apply to the same shape) or an fp16 hi and lo
-// part (XP = 2, ~2^-22).
+// part (XP = 2: an element to 2^-22, or 2^-25 in absolute terms if that is
+// more; rows scaled by a power of two to a largest magnitude of 2^8 to 2^9
+// where fp32 is replaced, so 2^-33 of the row's largest).
 //   NF4   xh.H + xh.R (+ xl.H), acc += absmax * (per 64 elements)
 //   Q4_0  B = q - 8, Q8_0 B = q: xh.B + xl.B, acc += d * (per 32 elements)
 //   Q4_K  B = q * sc: xh.B (+ xl.B), acc += d * (...); per super-block the

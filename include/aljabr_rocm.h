@@ -153,10 +153,13 @@ int aljabr_rocm_matvec_tb_q6_k(void *C, const void *A, const void *B, int K, int
 int aljabr_rocm_matvec_tb_q4_k_softcap(void *C, const void *A, const void *B, int K, int N, float cap);
 int aljabr_rocm_matvec_tb_q6_k_softcap(void *C, const void *A, const void *B, int K, int N, float cap);
 
-/* A[batchSize][K] fp32 -> C[batchSize][N] fp32 with W read once per call.
+/* A[batchSize][K] fp32 -> C[batchSize][N] fp32.
  * type: ALJABR_ROCM_TYPE_{Q4_0,Q8_0,Q4_K,Q6_K,F16}. Replaces aljabr_metal_matvec_tb_batch
- * (MTLC/aljabr_metal_matvec_api.h:93-94). batchSize < 16 runs the
- * wavefront-reduction kernels, batchSize >= 16 the MFMA kernels. */
+ * (MTLC/aljabr_metal_matvec_api.h:93-94). From batchSize 2 on the matrix cores
+ * where the shape allows (K % 512 == 0 for the quantized types), in passes over
+ * W of 8 (Q4_0, Q8_0) or 32 tokens, else in fp32 by 8; larger quantized batches,
+ * where that is faster, lay W out once for all tokens in the stream's scratch
+ * (at most 1 GiB; not while the stream is being captured). */
 int aljabr_rocm_matvec_tb_batch(void *C, const void *A, const void *B, int K,
                                 int N, int type, int batchSize);
 /* NF4 variant of the above (the Metal ABI has no NF4 batch entry). */
