@@ -317,3 +317,56 @@ def test_which_path(rocm, dev, oracle, t, ns, k, m, prompt):
     bytes_per = {Q4_0: 0.5625, Q8_0: 1.0625, Q4_K: 0.5625, Q6_K: 1.125, NF4: 0.5625}[t]
     image = min(sum(ns) * k * bytes_per, 100 << 20) + 2 * m * k
     assert (held >= image) == prompt, (held, image)
+
+
+@pytest.mark.parametrize("t,k,m", [(Q8_0, 9472, 130), (Q4_0, 1280, 700), (Q8_0, 2560, 300)])
+def test_infinite_activations_stay_infinite(rocm, dev, oracle, t, k, m):
+    """An infinity times a weight is infinite (NaN where the weight is zero)
+    through the folded sums and the slices; other tokens are not touched."""
+    n = 96
+    raw = _random_blocks(t, n, k, 3)
+    raw.reshape(-1, 18 if t == Q4_0 else 34)[:, 1] |= 4          # no zero scales
+    x = oracle.normal(4, m * k).reshape(m, k)
+    x[7, 70] = -np.inf
+    x[9, 3] = np.nan
+    y, w, xd = dev.empty(m * n), dev.put(raw), dev.put(x)
+    rocm.call("aljabr_rocm_matvec_tb_batch", dev.ptr(y), dev.ptr(xd), dev.ptr(w), k, n, t, m)
+    got = dev.get(y).reshape(m, n)
+    w64 = _decoded(oracle, t, raw.ravel(), n, k)
+    with np.errstate(invalid="ignore"):
+        want = -np.inf * np.sign(w64[:, 70])
+    assert np.array_equal(got[7], want, equal_nan=True)
+    assert np.isnan(got[9]).all()
+    rest = np.r_[0:7, 8, 10:m]
+    assert rel_l2(got[rest], x[rest].astype(np.float64) @ w64.T) <= TOL
+
+
+def test_captured_call_keeps_the_passes(rocm, dev, oracle):
+    """Under stream capture no scratch is taken: K % 512 != 0 runs in fp32 by 8
+    tokens, and every replay equals the oracle."""
+    import torch
+    t, n, k, m = Q8_0, 255, 640, 64
+    raw = _weights(oracle, t, n, k, 3)
+    x = oracle.normal(4, m * k).reshape(m, k)
+    w, xd, y = dev.put(raw), dev.put(x), dev.empty(m * n)
+    ref = x.astype(np.float64) @ _decoded(oracle, t, raw, n, k).T
+
+    def body():
+        stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+        rocm.call("aljabr_rocm_set_stream", stream.cuda_stream)
+        rocm.call("aljabr_rocm_set_sync_mode", 0)
+        with torch.cuda.graph(graph, stream=stream):
+            rocm.call("aljabr_rocm_matvec_tb_batch", dev.ptr(y), dev.ptr(xd), dev.ptr(w), k, n, t, m)
+        outs = []
+        for _ in range(3):
+            y.fill_(float("nan"))
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            outs.append(y.cpu().numpy().reshape(m, n))
+        return outs, scratch_held(rocm)
+
+    outs, held = fresh_thread(body)
+    assert held == 0
+    for got in outs:
+        assert rel_l2(got, ref) <= TOL
