@@ -466,10 +466,15 @@ namespace aljabr {
 //         14336 x 4096 17: 43/46, 18: 50/46     Q/K/V of 4096 17: 63/30
 //   Q8_0  2560 x 2560  16: 19/22, 17: 24/23     128256 x 4096 25: 495/504, 33: 624/508
 //         3328 x 1280   9: 27/18 (fp32)         Q/K/V of 2560  9: 38/23
-//   Q4_K  1024 x 1024  64: 17/18, 65: 19/18     4096 x 4096   66: 30/32, 97: 37/33
+//   Q4_K  Q/K/V of 4096 33: 43/31               2048 x 5632 twice (gate, up) 33: 33/27
 //         1280 x 1280   9: 10/17, 17: 18/17 (fp32)
-//   Q6_K  5632 x 2048  65: 32/33, 66: 35/32     14336 x 4096  65: 88/97, 66: 98/96
-//         3328 x 1280   9: 19/22, 16: 29/22 (fp32)
+//   Q6_K  3328 x 1280   9: 19/22, 16: 29/22 (fp32)
+// Where it is closer to float64 than the passes, these go to it whatever the
+// price: K-quants at K % 512 == 0 from 33 tokens (65 below 2 Mi and from 32 Mi
+// on; Q4_K 4.1e-7 -> 2.3e-7, Q6_K 1.9e-7 -> 1.2e-7), for up to a third more
+// time below 65 tokens (4096 x 4096 Q4_K 48: 20/27, 66: 30/32; 2560 x 2560 Q6_K
+// 48: 23/26), and Q4_0 and Q8_0 at other K below 32 Mi (3.6e-7 -> 1e-7; 512 x
+// 768 9: 10/14, 1280 x 1280 9: 15/15).
 namespace {
 
 float mega(int N, int K) { return static_cast<float>(N) * static_cast<float>(K) / (1 << 20); }
@@ -478,7 +483,8 @@ bool k_quant(int type) { return type == ALJABR_ROCM_TYPE_Q4_K || type == ALJABR_
 
 // One pass over an N x K matrix: 8 tokens in fp32 (K % 512 != 0), else on the
 // matrix cores 8 (Q4_0, Q8_0) or 32 (K-quants; their LDS-staged kernel's time
-// goes with the row tiles that its workgroups run in turn, kq_launch).
+// goes with the slices of 256 elements that its workgroups run in turn, see
+// kq_launch).
 float pass_us(int type, int N, int K, int xparts) {
     const float mi = mega(N, K);
     if (K % 512 != 0)
@@ -488,14 +494,14 @@ float pass_us(int type, int N, int K, int xparts) {
     if (type == ALJABR_ROCM_TYPE_Q4_K && xparts == 1) return 8.0f + 0.235f * mi;
     const bool q4 = type == ALJABR_ROCM_TYPE_Q4_K;
     const long long cus = device_cu_count() > 0 ? device_cu_count() : 256;
-    const long long units = (N + 127LL) / 128 * (K / 512);
-    const bool one = units <= cus;               // one row tile a workgroup
+    const long long units = (N + 255LL) / 256 * (K / 512);
+    const bool one = 2 * units <= cus;           // a workgroup has one slice of 256
     if (type == ALJABR_ROCM_TYPE_Q4_0) return one ? 7.5f + 0.07f * mi : 8.0f + 0.18f * mi;
     if (type == ALJABR_ROCM_TYPE_Q8_0) return one ? 8.2f + 0.12f * mi : 10.5f + 0.19f * mi;
     if (one) return q4 ? 8.0f + 0.2f * mi : 10.0f + 0.15f * mi;
-    const long long nt = (units + 1) / 2 <= cus || !q4 ? 2 : 4;
-    const float tiles = static_cast<float>(((units + nt - 1) / nt + cus - 1) / cus * nt);
-    return q4 ? 1.5f + 7.0f * tiles : 5.0f + 7.7f * tiles;
+    const long long nt = units <= cus ? 1 : (units + 1) / 2 <= cus || !q4 ? 2 : 4;
+    const float halves = static_cast<float>(2 * nt * (((units + nt - 1) / nt + cus - 1) / cus));
+    return q4 ? 1.5f + 7.0f * halves : 5.0f + 7.7f * halves;
 }
 
 // Passes for M tokens; a last single token takes the batch-1 kernel.
@@ -528,11 +534,14 @@ bool prompt_gguf(int type, int M, const int *N, int n, int K, int xparts) {
     // One pass takes them all, in one launch for a stack.
     if (M <= (K % 512 == 0 && k_quant(type) ? 32 : 8)) return false;
     float passes = 0.0f, mi = 0.0f;
+    bool accurate = (K % 512 == 0) == k_quant(type);
     for (int i = 0; i < n; ++i) {
+        const float size = mega(N[i], K);
         passes += pass_us(type, N[i], K, xparts);
-        mi += mega(N[i], K);
+        mi += size;
+        accurate = accurate && (k_quant(type) ? M > (size >= 32.0f || size < 2.0f ? 64 : 32) : size < 32.0f);
     }
-    return pass_count(type, M, K) * passes > prompt_us(type, M, mi, xparts);
+    return accurate || pass_count(type, M, K) * passes > prompt_us(type, M, mi, xparts);
 }
 
 // NF4: passes of 64. At K of 1024 and multiples of 4096 and N > 2 K (gate, up)

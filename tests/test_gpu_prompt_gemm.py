@@ -287,9 +287,9 @@ def test_prompt_token_passes(rocm, dev, oracle, m):
 # matrices and stacks.
 @pytest.mark.parametrize("t,ns,k,m,prompt", [
     (Q4_0, (4096,), 4096, 17, False), (Q4_0, (4096,), 4096, 25, True), (Q8_0, (4096,), 4096, 9, False),
-    (Q4_0, (4096, 1024, 1024), 4096, 9, True), (Q8_0, (2560, 640, 640), 2560, 17, True), (Q8_0, (1280,), 1280, 9, False),
-    (Q8_0, (3328,), 1280, 9, True), (Q4_K, (4096,), 4096, 64, False), (Q4_K, (4096,), 4096, 98, True),
-    (Q4_K, (1024,), 2048, 33, False), (Q4_K, (1024,), 1024, 66, True), (Q4_K, (4096, 1024, 1024), 4096, 66, True),
+    (Q4_0, (4096, 1024, 1024), 4096, 9, True), (Q8_0, (2560, 640, 640), 2560, 17, True), (Q8_0, (1280,), 1280, 9, True), (Q8_0, (2560,), 2560, 9, False),
+    (Q8_0, (3328,), 1280, 9, True), (Q4_K, (4096,), 4096, 32, False), (Q4_K, (4096,), 4096, 33, True),
+    (Q4_K, (1024,), 1536, 64, False), (Q4_K, (1024,), 1024, 66, True), (Q4_K, (4096, 1024, 1024), 4096, 66, True),
     (Q6_K, (1024,), 1024, 33, False), (Q6_K, (1024,), 1024, 66, True), (Q6_K, (3328,), 1280, 24, True),
     (NF4, (4096,), 4096, 128, False), (NF4, (4096,), 4096, 160, True), (NF4, (14336,), 4096, 160, False),
     (NF4, (640,), 2560, 66, True)])
