@@ -594,11 +594,10 @@ __global__ __launch_bounds__(kPgThreads, (PgLds<F, XP, MT, NT>::kSimdWaves)) voi
     // only (half of that in short slices): one fp32 chain over all of K rounds
     // more than the waves and slices of the passes do. Error against float64 of
     // the passes, one chain, this: Q8_0 4096 x 14336, 512 tokens 1.18e-7,
-    // 2.08e-7, 1.10e-7; K = 1024 0.98, 1.25, 0.94. What the other formats
-    // replace rounds more (1.8e-7 to 4.1e-7): half as many folds. They cost 2
-    // to 8 % of the time at four token tiles. One part is rounded to 2e-4
-    // anyway: none.
-    constexpr int kFold = F == kPgQ40 || F == kPgQ80 ? 8 : 16;
+    // 2.08e-7, 1.10e-7; K = 1024 0.98, 1.25, 0.94. The passes of NF4 and Q6_K
+    // round more (1.9e-7 to 2.1e-7): half as many folds. They cost 2 to 8 % of
+    // the time at four token tiles. One part is rounded to 2e-4 anyway: none.
+    constexpr int kFold = F == kPgNF4 || F == kPgQ6K ? 16 : 8;
     const int step = XP == 1 ? a.chunks : kb1 - kb0 <= 2 * kFold ? kFold / 2 : kFold;
     f32x16 tot[MT][NT];
 #pragma unroll
