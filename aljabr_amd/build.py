@@ -1,9 +1,8 @@
 """Build recipe for libaljabr_rocm.so (gfx950 only).
 
 Compiles every ``csrc/*.hip`` file with hipcc into ``_build/`` and links the C
-ABI library next to this file. Run ``python -m aljabr_amd.build``; the round
-driver calls it through ``__graft_entry__.build()``. Cross-compiles without a
-GPU.
+ABI library next to this file: ``python -m aljabr_amd.build``. Cross-compiles
+without a GPU.
 """
 from __future__ import annotations
 
