@@ -31,7 +31,8 @@ DEVICE_FLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-m
                 "-amdgpu-kernarg-preload-count=14"]
 # The prompt GEMM runs one wave per SIMD. There the compiler would put the
 # matrix products in AGPRs, which the vector ALU cannot read without a copy of
-# each (Q4_K_M FFN, 2048 tokens: 2.13 ms so, 1.48 ms with them in VGPRs).
+# each (FFN 4096 x 14336, Q4_K_M, 2048 tokens: 1.67 ms so, 1.49 ms with them in
+# VGPRs; Q8_0, 512 tokens: 588 and 534 us).
 FILE_FLAGS = {f"prompt_{t}.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"] for t in ("nf4", "q40", "q80", "q4k", "q6k")}
 COMMON = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-Wall", "-Wno-unused-function"]
 
